@@ -99,10 +99,11 @@ __device__ __forceinline__ void amr_item(const AmrPassArgsT<Real>& pa, long long
                 for (int q = 0; q < 5; ++q) u[q] = a.G[amr_g(a, q, slot, s, layer, t)];
             }
         }
-        to_prim(e, u, wv);
+        Real v;
+        to_prim_v(e, u, wv, v);
 #pragma unroll
         for (int q = 0; q < 5; ++q) sw[q][c][p] = wv[q];
-        sre[c][p] = eos_rho_e(e, wv[0], wv[4]);
+        sre[c][p] = eos_rho_e_v(e, wv[0], wv[4], v);
         if constexpr (HYB) {
             ss[0][c][p] = log(fmax(wv[0], Real(1e-300)));
             ss[1][c][p] = log(fmax(wv[4] + e.p_inf, Real(1e-300)));
@@ -111,7 +112,8 @@ __device__ __forceinline__ void amr_item(const AmrPassArgsT<Real>& pa, long long
     __syncthreads();
     // amr.rs:1254; formed in double from the device dt and rounded to Real
     const double lam = pa.ndim_pos > 0.0 ? pa.ndim_pos * dtv / (double)dx : 0.0;
-    tile_faces<D, MODE, B, P, NT>(sw, sre, sm, ss, sth, B, Pv, 0, B, e, Real(lam), pa.tol, n_shock, n_fb, n_lim);
+    tile_faces<D, MODE, B, P, NT>(sw, sre, sm, ss, sth, B, Pv, 0, B, e, Real(lam), pa.tol, a.bd[(D + 1) % 3] == 1,
+                                 a.bd[(D + 2) % 3] == 1, n_shock, n_fb, n_lim);
     // ---- residual and boundary face fluxes
     for (int it = tid; it < B * P; it += NT) {
         int c, p;

@@ -18,11 +18,14 @@
 
 #include <cstdint>
 
+#include "em_div.h"
+
 namespace em {
 
 template <class R>
 struct EosT {
     R gamma, p_inf, b, q;
+    R rg = R(1) / (gamma - R(1));  // correctly rounded reciprocal, for div_by
 };
 using Eos = EosT<double>;
 
@@ -107,17 +110,74 @@ __device__ __forceinline__ void phys_flux(const R w[5], const R q[5], R f[5]) {
     f[4] = (q[4] + w[4]) * u;
 }
 
-// HLLC with Davis wave-speed bounds: system.rs:260-312.  Returns the flux.
+// to_prim, its divisions by rho through one reciprocal; v = 1 / rho.  (The
+// float variant keeps the plain forms throughout: its results on flat
+// sub-stencils hang on the contracted expressions' last bits.)
+template <class R>
+__device__ __forceinline__ void to_prim_v(const EosT<R>& e, const R u[5], R w[5], R& v) {
+    const R rho = u[0];
+    if constexpr (sizeof(R) == 4) {
+        to_prim(e, u, w);
+        v = R(1.0) / rho;
+    } else {
+        const R r = rcp_mid(rho);
+        v = inv_by(rho, r);
+        const R vx = div_by(u[1], rho, r), vy = div_by(u[2], rho, r), vz = div_by(u[3], rho, r);
+        const R en = div_by(u[4], rho, r) - R(0.5) * (vx * vx + vy * vy + vz * vz);
+        w[0] = rho;
+        w[1] = vx;
+        w[2] = vy;
+        w[3] = vz;
+        w[4] = (e.gamma - R(1.0)) * (en - e.q) / (v - e.b) - e.gamma * e.p_inf;
+        // an overflowing quotient leaves p infinite or NaN
+        if (!in_mid(rho) || too_small(u[1]) || too_small(u[2]) || too_small(u[3]) || too_small(u[4]) ||
+            !(fabs(w[4]) <= Mid<R>::huge)) {
+            to_prim(e, u, w);
+            v = R(1.0) / rho;
+        }
+    }
+}
+// eos_rho_e with v = 1 / rho given and the division by the constant
+// gamma - 1 through its reciprocal.
+template <class R>
+__device__ __forceinline__ R eos_rho_e_v(const EosT<R>& e, R rho, R p, R v) {
+    if constexpr (sizeof(R) == 4) {
+        return eos_rho_e(e, rho, p);
+    } else {
+        const R a = (p + e.gamma * e.p_inf) * (v - e.b);
+        R x = div_by(a, e.gamma - R(1.0), e.rg);
+        if (too_small(a) || !(fabs(x) <= Mid<R>::huge)) x = a / (e.gamma - R(1.0));
+        return rho * (x + e.q);
+    }
+}
+
+// True where the conserved state q is admissible with so much room that the
+// rounded evaluation (to_prim, then admissible) cannot decide otherwise, and
+// is finite; no division.  With d = (E - |m|^2 / 2 rho - rho q - p_inf (1 -
+// rho b)) rho = rho^2 (v - b) (p + p_inf) / (gamma - 1), the test asks for
+// d > margin times the sum of the terms' magnitudes; the rounding of either
+// evaluation is below 1e-5 of that slack.
+template <class R>
+__device__ __forceinline__ bool clearly_admissible(const EosT<R>& e, const R q[5]) {
+    const R rho = q[0];
+    const R a = rho * q[4], k = R(0.5) * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
+    const R rb = rho * e.b;
+    const R y = rho * (rho * e.q), z = rho * e.p_inf * (R(1.0) - rb);
+    const R d = a - k - y - z;
+    const R size = fabs(a) + k + fabs(y) + fabs(z);
+    return in_mid(rho) && fabs(rb) <= R(0.5) && d > Mid<R>::margin * size && d > Mid<R>::lo * Mid<R>::lo &&
+           size < Mid<R>::hi * Mid<R>::hi && e.rg > R(0.0) && e.rg < R(100.0);
+}
+
+// The flux and the selected star state of HLLC once the two sound speeds
+// and conserved states are known (system.rs:268-312).
 template <int D, class R>
-__device__ __forceinline__ void hllc(const EosT<R>& e, const R wl[5], const R wr[5], R f[5]) {
+__device__ __forceinline__ void hllc_flux(const R wl[5], const R wr[5], const R ql[5], const R qr[5], R cl, R cr,
+                                          R f[5]) {
     constexpr int un = 1 + D;
-    R cl = sound_speed(e, wl[0], wl[4]), cr = sound_speed(e, wr[0], wr[4]);
     R ul = wl[un], ur = wr[un];
     R sl = fmin(ul - cl, ur - cr);
     R sr = fmax(ul + cl, ur + cr);
-    R ql[5], qr[5];
-    to_cons(e, wl, ql);
-    to_cons(e, wr, qr);
     if (sl >= R(0.0)) {
         phys_flux<D>(wl, ql, f);
         return;
@@ -151,6 +211,16 @@ __device__ __forceinline__ void hllc(const EosT<R>& e, const R wl[5], const R wr
     phys_flux<D>(w, q, fw);
 #pragma unroll
     for (int k = 0; k < 5; ++k) f[k] = fw[k] + s * (qs[k] - q[k]);
+}
+
+// HLLC with Davis wave-speed bounds: system.rs:260-312.  Returns the flux.
+template <int D, class R>
+__device__ __forceinline__ void hllc(const EosT<R>& e, const R wl[5], const R wr[5], R f[5]) {
+    const R cl = sound_speed(e, wl[0], wl[4]), cr = sound_speed(e, wr[0], wr[4]);
+    R ql[5], qr[5];
+    to_cons(e, wl, ql);
+    to_cons(e, wr, qr);
+    hllc_flux<D>(wl, wr, ql, qr, cl, cr, f);
 }
 
 // KEEP-PE two-point flux: system.rs:317-334
@@ -279,6 +349,168 @@ __device__ __forceinline__ bool midpoint_flux(const EosT<R>& e, const R (&s)[6][
     }
     hllc<D>(e, wl, wr, f);
     return fb;
+}
+
+// Both WENO5-Z interpolations of a midpoint's six point values, left (v0..v4)
+// and right (v5, v4, .., v1): the values weno5z_interp gives, with fewer
+// operations and no range scaling.
+//   * 2x, 4x and x/4 are exact, so a sum with them is one fma with the same
+//     rounding; 6x = 2 (3x) and 10x = 2 (5x) share their products.  The
+//     contracted build (EM_CONTRACT) keeps weno5z_interp's expressions, whose
+//     fused rounding residues keep beta above zero on flat stencils.
+//   * The factor 1/8 of the candidates and 1/16 of the linear weights
+//     (1, 10, 5)/16 are powers of two: the weighted sum is formed without
+//     them and scaled once.
+//   * tau / (beta + eps): the reciprocals of the three (rcp3_mid), and of the
+//     two weight sums (rcp2_mid), are taken jointly.  A tau too small for the
+//     core leaves 1 + r^2 = 1 either way.
+// top is raised to the largest beta's high word, ok cleared where the last
+// quotient needs the general division: the caller falls back to
+// weno5z_interp unless ok and top below beta_max.  95 issue slots a side (a
+// reciprocal counts four) against about 125.
+__device__ __forceinline__ void weno5z_pair(const double v[6], double& left, double& right, unsigned& top, bool& ok) {
+#ifndef EM_CONTRACT
+    const double m0 = 3.0 * v[0], m2 = 3.0 * v[2], m3 = 3.0 * v[3], m5 = 3.0 * v[5];
+    const double f1 = 5.0 * v[1], f4 = 5.0 * v[4];
+#endif
+    const double c13 = 13.0 / 12.0;
+    double N[2], S[2];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const double a = s ? v[5] : v[0], b = s ? v[4] : v[1], c = s ? v[3] : v[2], d = s ? v[2] : v[3], g = s ? v[1] : v[4];
+#ifndef EM_CONTRACT
+        const double ma = s ? m5 : m0, mc = s ? m3 : m2, md = s ? m2 : m3, fb = s ? f4 : f1;
+        const double q0 = __builtin_fma(-2.0, fb, ma) + 15.0 * c;
+        const double q1 = __builtin_fma(2.0, mc, -b) + md;
+        const double q2 = __builtin_fma(2.0, md, mc) - g;
+        const double t0 = __builtin_fma(-2.0, b, a) + c, s0 = __builtin_fma(-4.0, b, a) + mc;
+        const double t1 = __builtin_fma(-2.0, c, b) + d, s1 = b - d;
+        const double t2 = __builtin_fma(-2.0, d, c) + g, s2 = __builtin_fma(-4.0, d, mc) + g;
+        const double b0 = __builtin_fma(0.25, s0 * s0, c13 * (t0 * t0));
+        const double b1 = __builtin_fma(0.25, s1 * s1, c13 * (t1 * t1));
+        const double b2 = __builtin_fma(0.25, s2 * s2, c13 * (t2 * t2));
+#else
+        const double q0 = 3.0 * a - 10.0 * b + 15.0 * c;
+        const double q1 = -b + 6.0 * c + 3.0 * d;
+        const double q2 = 3.0 * c + 6.0 * d - g;
+        const double t0 = a - 2.0 * b + c, s0 = a - 4.0 * b + 3.0 * c;
+        const double t1 = b - 2.0 * c + d, s1 = b - d;
+        const double t2 = c - 2.0 * d + g, s2 = 3.0 * c - 4.0 * d + g;
+        const double b0 = c13 * (t0 * t0) + 0.25 * (s0 * s0);
+        const double b1 = c13 * (t1 * t1) + 0.25 * (s1 * s1);
+        const double b2 = c13 * (t2 * t2) + 0.25 * (s2 * s2);
+#endif
+        const double tau = fabs(b0 - b2);
+        const double d0 = b0 + 1e-40, d1 = b1 + 1e-40, d2 = b2 + 1e-40;
+        top = max(max(top, top_word(d0)), max(top_word(d1), top_word(d2)));
+        double i0, i1, i2;
+        rcp3_mid(d0, d1, d2, i0, i1, i2);
+        const double r0 = div_by(tau, d0, i0), r1 = div_by(tau, d1, i1), r2 = div_by(tau, d2, i2);
+        const double a0 = 1.0 + r0 * r0;
+        const double a1 = 10.0 * (1.0 + r1 * r1);
+        const double a2 = 5.0 * (1.0 + r2 * r2);
+        N[s] = a0 * q0 + a1 * q1 + a2 * q2;
+        S[s] = a0 + a1 + a2;
+    }
+    double il, ir;
+    rcp2_mid(S[0], S[1], il, ir);
+    const double ql = div_by_fix(N[0], S[0], il), qr = div_by_fix(N[1], S[1], ir);
+    ok = ok && (fabs(ql) >= Mid<double>::tiny || N[0] == 0.0) && (fabs(qr) >= Mid<double>::tiny || N[1] == 0.0);
+    left = 0.125 * ql;
+    right = 0.125 * qr;
+}
+
+// midpoint_flux for operands in the middle of the exponent range, stencil
+// value k of cell j read through ld(j, k): the same flux, or false (and no
+// flux) where some operand is outside, or a reconstruction inadmissible: the
+// caller then evaluates midpoint_flux.  The pass is bound by its FP64
+// instruction count (VALU 87% busy), much of it divisions: 61 per midpoint,
+// here 6 in the general form and the rest through shared reciprocals.  With
+// the load phase's and the limiter's divisions (to_prim_v,
+// clearly_admissible) the 256^3 Weno x pass went from 2,544 to 2,033 VALU
+// instructions per cell, the three passes from 4.29 to 3.56 ms.
+//   * l4un = -l0un and l44 = l04 = -l14 / 2 exactly (powers of two and signs),
+//     so the fields 0, 1 and 4 need two products per cell.
+//   * zero1, zero2: the axes of the transverse velocities t1, t2 are
+//     inactive (uniform); where such a component is +0 on the whole wave its
+//     reconstructions are +0 and are not evaluated.
+template <int D, class LD>
+__device__ __forceinline__ bool midpoint_flux_mid(const Eos& e, bool zero1, bool zero2, LD&& ld, double f[5]) {
+    constexpr int un = 1 + D;
+    constexpr int t1 = 1 + (D + 1) % 3;
+    constexpr int t2 = 1 + (D + 2) % 3;
+    const double rho = 0.5 * (ld(2, 0) + ld(3, 0));
+    const double avp = 0.5 * (ld(2, 4) + ld(3, 4));
+    const double irho = rcp_mid(rho);
+    const double v = inv_by(rho, irho);
+    const double vb = v - e.b;
+    const double c2 = div_by(e.gamma * (avp + e.p_inf) * v * v, vb, rcp_mid(vb));
+    bool ok = in_mid(rho) && in_mid(vb) && in_mid(c2) && e.rg > 0.0 && e.rg <= Mid<double>::hi;
+    const double c = sqrt_mid(c2);
+    const double cc = c * c;
+    const double lu = 0.5 * div_by(rho, c, rcp_mid(c));  // rho / (2 c)
+    const double lp = 0.5 * inv_by(cc, rcp_mid(cc));     // 1 / (2 c^2)
+    const double ru = div_by(c, rho, irho);                 // c / rho
+    unsigned top = 0;
+    double wl[5], wr[5];
+    {
+        double ch[6], l0, r0, l1, r1, l4, r4;
+#pragma unroll
+        for (int j = 0; j < 6; ++j) ch[j] = lp * ld(j, 4) - lu * ld(j, un);
+        weno5z_pair(ch, l0, r0, top, ok);
+#pragma unroll
+        for (int j = 0; j < 6; ++j) ch[j] = lp * ld(j, 4) + lu * ld(j, un);
+        weno5z_pair(ch, l4, r4, top, ok);
+#pragma unroll
+        for (int j = 0; j < 6; ++j)
+#ifndef EM_CONTRACT
+            ch[j] = __builtin_fma(-2.0, lp * ld(j, 4), ld(j, 0));
+#else
+            ch[j] = ld(j, 0) - 2.0 * lp * ld(j, 4);
+#endif
+        weno5z_pair(ch, l1, r1, top, ok);
+        wl[0] = l0 + l1 + l4;
+        wr[0] = r0 + r1 + r4;
+        wl[un] = ru * l4 - ru * l0;
+        wr[un] = ru * r4 - ru * r0;
+        wl[4] = cc * l0 + cc * l4;
+        wr[4] = cc * r0 + cc * r4;
+    }
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const int t = s ? t2 : t1;
+        double ch[6];
+#pragma unroll
+        for (int j = 0; j < 6; ++j) ch[j] = ld(j, t);
+        wl[t] = wr[t] = 0.0;
+        if (!(s ? zero2 : zero1) || __any(any_bits(ch[0], ch[1], ch[2]) | any_bits(ch[3], ch[4], ch[5])))
+            weno5z_pair(ch, wl[t], wr[t], top, ok);
+    }
+    // both states admissible, with sound speeds in range
+    const double il = rcp_mid(wl[0]), ir = rcp_mid(wr[0]);
+    const double vl = inv_by(wl[0], il), vr = inv_by(wr[0], ir);
+    const double vbl = vl - e.b, vbr = vr - e.b;
+    const double c2l = div_by(e.gamma * (wl[4] + e.p_inf) * vl * vl, vbl, rcp_mid(vbl));
+    const double c2r = div_by(e.gamma * (wr[4] + e.p_inf) * vr * vr, vbr, rcp_mid(vbr));
+    ok = ok && top < top_word(Mid<double>::beta_max) && in_mid(wl[0]) && in_mid(wr[0]) && in_mid(vbl) && in_mid(vbr) &&
+         in_mid(c2l) && in_mid(c2r) && wl[4] + e.p_inf > 0.0 && wr[4] + e.p_inf > 0.0;
+    double ql[5], qr[5];
+#pragma unroll
+    for (int s = 0; s < 2; ++s) {
+        const double* w = s ? wr : wl;
+        double* q = s ? qr : ql;
+        const double ke = 0.5 * w[0] * (w[1] * w[1] + w[2] * w[2] + w[3] * w[3]);
+        q[0] = w[0];
+        q[1] = w[0] * w[1];
+        q[2] = w[0] * w[2];
+        q[3] = w[0] * w[3];
+        const double a = (w[4] + e.gamma * e.p_inf) * (s ? vbr : vbl);
+        ok = ok && !too_small(a);
+        q[4] = w[0] * (div_by(a, e.gamma - 1.0, e.rg) + e.q) + ke;
+    }
+    if (!ok) return false;
+    hllc_flux<D>(wl, wr, ql, qr, sqrt_mid(c2l), sqrt_mid(c2r), f);
+    return true;
 }
 
 // Flux-form weights of the 6th-order midpoint-to-node difference:

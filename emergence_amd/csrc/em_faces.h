@@ -12,6 +12,8 @@
 // barrier): sm[k][f][p] holds the flux of face f = 0 .. Tv (between cells
 // c0+f-1 and c0+f).  Counters of midpoints and faces
 // owned by the tile (tiles of one pencil share their halo) are accumulated.
+// zero1, zero2: the axes of the transverse velocities (D+1) % 3 and
+// (D+2) % 3 are inactive (see midpoint_flux_mid).
 #pragma once
 #include "em_device.h"
 #include "em_types.h"
@@ -24,7 +26,7 @@ __device__ __forceinline__ void tile_faces(R (&sw)[5][T + 10][P], R (&sre)[T + 1
                                            R (&sm)[5][T + 5][P],
                                            R (&ss)[2][MODE == MODE_HYBRID ? T + 10 : 1][P],
                                            R (&sth)[MODE == MODE_HYBRID ? T + 1 : 1][P], int Tv, int Pv,
-                                           int c0, int nD, const EosT<R>& e, R lam, R tol,
+                                           int c0, int nD, const EosT<R>& e, R lam, R tol, bool zero1, bool zero2,
                                            unsigned& n_shock, unsigned& n_fb, unsigned& n_lim) {
     constexpr int M = T + 5;
     constexpr int NF = T + 1;
@@ -65,13 +67,18 @@ __device__ __forceinline__ void tile_faces(R (&sw)[5][T + 10][P], R (&sre)[T + 1
                 for (int f = flo; f <= fhi; ++f) need = need || sth[f][p] > R(0.0);
                 if (!need) continue;
             }
-            R s[6][5];
-#pragma unroll
-            for (int j = 0; j < 6; ++j)
-#pragma unroll
-                for (int k = 0; k < 5; ++k) s[j][k] = sw[k][m + j][p];
             R f[5];
-            const bool fb = midpoint_flux<D>(e, s, f);
+            bool fb = false, done = false;
+            if constexpr (sizeof(R) == 8)
+                done = midpoint_flux_mid<D>(e, zero1, zero2, [&](int j, int k) { return sw[k][m + j][p]; }, f);
+            if (!done) {
+                R s[6][5];
+#pragma unroll
+                for (int j = 0; j < 6; ++j)
+#pragma unroll
+                    for (int k = 0; k < 5; ++k) s[j][k] = sw[k][m + j][p];
+                fb = midpoint_flux<D>(e, s, f);
+            }
 #pragma unroll
             for (int k = 0; k < 5; ++k) sm[k][m][p] = f[k];
             if (fb) {
@@ -155,21 +162,32 @@ __device__ __forceinline__ void tile_faces(R (&sw)[5][T + 10][P], R (&sre)[T + 1
             phys_flux<D>(wl, ul, fl);
             phys_flux<D>(wr, ur, fr);
             const R tl = R(2.0) * lam;
-            auto ok = [&](const R* fx) {
-                R qa[5], qb[5], pa[5], pb[5];
+            R qa[5], qb[5];
+            auto test_states = [&](const R* fx) {
 #pragma unroll
                 for (int k = 0; k < 5; ++k) {
                     qa[k] = ul[k] - tl * (fx[k] - fl[k]);
                     qb[k] = ur[k] + tl * (fx[k] - fr[k]);
                 }
+            };
+            auto ok = [&](const R* fx) {
+                R pa[5], pb[5];
+                test_states(fx);
                 to_prim(e, qa, pa);
                 to_prim(e, qb, pb);
                 return admissible(e, pa[0], pa[4]) && admissible(e, pb[0], pb[4]);
             };
-            bool fin = true;
+            // almost every face is admissible by a wide margin, which needs
+            // no division to see (a non-finite flux never passes)
+            test_states(fo);
+            bool pass = clearly_admissible(e, qa) && clearly_admissible(e, qb);
+            if (!pass) {
+                pass = true;
 #pragma unroll
-            for (int k = 0; k < 5; ++k) fin = fin && isfinite(fo[k]);
-            if (!(fin && ok(fo))) {
+                for (int k = 0; k < 5; ++k) pass = pass && isfinite(fo[k]);
+                pass = pass && ok(fo);
+            }
+            if (!pass) {
                 constexpr int un = 1 + D;
                 const R al = fmax(fabs(wl[un]) + sound_speed(e, wl[0], wl[4]),
                                        fabs(wr[un]) + sound_speed(e, wr[0], wr[4]));

@@ -145,10 +145,11 @@ __device__ __forceinline__ void axis_tile(const PassArgsT<Real>& a, int bid, Til
         } else {
             ghost_state<D>(a, pen, g, u);
         }
-        to_prim(e, u, w);
+        Real v;
+        to_prim_v(e, u, w, v);
 #pragma unroll
         for (int k = 0; k < 5; ++k) sw[k][c][p] = w[k];
-        sre[c][p] = eos_rho_e(e, w[0], w[4]);
+        sre[c][p] = eos_rho_e_v(e, w[0], w[4], v);
         if constexpr (HYB) {
             // Euler::sensor, system.rs:409-413
             ss[0][c][p] = log(fmax(w[0], Real(1e-300)));
@@ -163,7 +164,8 @@ __device__ __forceinline__ void axis_tile(const PassArgsT<Real>& a, int bid, Til
         const double dt = a.stage_dt_host ? a.stage_dt : a.sc->dt;
         lam = a.ndim_pos * dt / a.dx_d;  // solver.rs:393
     }
-    tile_faces<D, MODE, T, P, NT>(sw, sre, sm, ss, sth, Tv, Pv, c0, nD, e, Real(lam), a.tol, n_shock, n_fb, n_lim);
+    tile_faces<D, MODE, T, P, NT>(sw, sre, sm, ss, sth, Tv, Pv, c0, nD, e, Real(lam), a.tol,
+                                 !a.active[(D + 1) % 3], !a.active[(D + 2) % 3], n_shock, n_fb, n_lim);
 
     // ---- 5. divergence, fused RK stage and CFL rate
     double rate = 0.0;

@@ -20,33 +20,23 @@ namespace EM_VARIANT {
 
 // LDS of one work item (whole pencils of a B-cell block, P of them)
 template <class Real, int MODE, int B, int P>
-struct AmrLds {
-    static constexpr bool HYB = MODE == MODE_HYBRID;
-    Real sw[5][B + 10][P];
-    Real sre[B + 10][P];  // rho_e of each cell
-    Real sm[5][B + 5][P];
-    Real ss[2][HYB ? B + 10 : 1][P];
-    Real sth[HYB ? B + 1 : 1][P];
-};
+using AmrLds = Tile<Real, MODE, B, P, false>;
 
 // Work item w of one batched AMR pass: the pencil group w % ngroup of leaf
 // leaf0 + w / ngroup (every thread of the workgroup calls it; it returns
-// after a barrier).  Counters of shock-path faces, fallbacks and limited
-// faces are added to the calling thread's n_*.
+// after a barrier).  Shock-path faces are added to the calling wave's n_shock,
+// fallbacks and limited faces to scnt.
 template <int D, int MODE, int B, int P, int NT, class Real>
 __device__ __forceinline__ void amr_item(const AmrPassArgsT<Real>& pa, long long w, AmrLds<Real, MODE, B, P>& L,
-                                         unsigned& n_shock, unsigned& n_fb, unsigned& n_lim) {
+                                         unsigned& n_shock, unsigned (&scnt)[3]) {
     constexpr int C = B + 10;
     constexpr bool HYB = MODE == MODE_HYBRID;
     constexpr int E0 = D == 0 ? 1 : 0;
     constexpr int E1 = D == 2 ? 1 : 2;
-    auto& sw = L.sw;
-    auto& sre = L.sre;
+    using TL = AmrLds<Real, MODE, B, P>;
     auto& sm = L.sm;
-    auto& ss = L.ss;
-    auto& sth = L.sth;
     const AmrDevT<Real>& a = pa.a;
-    const int tid = threadIdx.x;
+    const int tid = opaque(threadIdx.x);  // as in axis_segment
     const int be1 = a.bd[E1];
     const int nt = a.bcells / B;  // pencils of a block along D
     const int ngh = a.ng;
@@ -102,18 +92,18 @@ __device__ __forceinline__ void amr_item(const AmrPassArgsT<Real>& pa, long long
         Real v;
         to_prim_v(e, u, wv, v);
 #pragma unroll
-        for (int q = 0; q < 5; ++q) sw[q][c][p] = wv[q];
-        sre[c][p] = eos_rho_e_v(e, wv[0], wv[4], v);
+        for (int q = 0; q < 5; ++q) L.sw[q][TL::at(c, p)] = wv[q];
+        L.sre[TL::at(c, p)] = eos_rho_e_v(e, wv[0], wv[4], v);
         if constexpr (HYB) {
-            ss[0][c][p] = log(fmax(wv[0], Real(1e-300)));
-            ss[1][c][p] = log(fmax(wv[4] + e.p_inf, Real(1e-300)));
+            L.ss[0][TL::at(c, p)] = log(fmax(wv[0], Real(1e-300)));
+            L.ss[1][TL::at(c, p)] = log(fmax(wv[4] + e.p_inf, Real(1e-300)));
         }
     }
     __syncthreads();
     // amr.rs:1254; formed in double from the device dt and rounded to Real
     const double lam = pa.ndim_pos > 0.0 ? pa.ndim_pos * dtv / (double)dx : 0.0;
-    tile_faces<D, MODE, B, P, NT>(sw, sre, sm, ss, sth, B, Pv, 0, B, e, Real(lam), pa.tol, a.bd[(D + 1) % 3] == 1,
-                                 a.bd[(D + 2) % 3] == 1, n_shock, n_fb, n_lim);
+    tile_faces<D, MODE, NT>(L, tid, true, B, Pv, 0, 0, B, B, e, Real(lam), pa.tol, a.bd[(D + 1) % 3] == 1,
+                            a.bd[(D + 2) % 3] == 1, n_shock, scnt, [] {});
     // ---- residual and boundary face fluxes
     for (int it = tid; it < B * P; it += NT) {
         int c, p;
@@ -135,7 +125,8 @@ __device__ __forceinline__ void amr_item(const AmrPassArgsT<Real>& pa, long long
         for (int q = 0; q < 5; ++q) {
             const long long ix = amr_u(a, q, slot, cell);
             const Real prev = pa.first ? Real(0.0) : a.R[ix];
-            a.R[ix] = prev - (sm[q][c + 1][p] - sm[q][c][p]) / dx;
+            const Real fl = c == 0 ? L.sf[q][p] : sm[q][TL::mt(c - 1, p)];
+            a.R[ix] = prev - (sm[q][TL::mt(c, p)] - fl) / dx;
         }
     }
     for (int it = tid; it < 2 * P; it += NT) {
@@ -143,7 +134,7 @@ __device__ __forceinline__ void amr_item(const AmrPassArgsT<Real>& pa, long long
         if (p >= Pv) continue;
         const int t = t0 + p;
 #pragma unroll
-        for (int q = 0; q < 5; ++q) a.F[amr_f(a, q, slot, 2 * D + side, t)] = sm[q][side ? B : 0][p];
+        for (int q = 0; q < 5; ++q) a.F[amr_f(a, q, slot, 2 * D + side, t)] = side ? sm[q][TL::mt(B - 1, p)] : L.sf[q][p];
     }
     __syncthreads();
 }
@@ -158,20 +149,13 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(EM_WAVES_PER
     const int tid = threadIdx.x;
     if (tid < 3) scnt[tid] = 0;
     const long long nwork = (long long)pa.nleaves * pa.ngroup;
-    unsigned int n_shock = 0, n_fb = 0, n_lim = 0;
+    unsigned int n_shock = 0;
+    __syncthreads();
     // plain stride: the chunked XCD order (xcd_stride) measured no faster here
     for (long long w = blockIdx.x; w < nwork; w += gridDim.x)
-        amr_item<D, MODE, B, P, NT>(pa, w, L, n_shock, n_fb, n_lim);
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        n_shock += __shfl_xor(n_shock, off);
-        n_fb += __shfl_xor(n_fb, off);
-        n_lim += __shfl_xor(n_lim, off);
-    }
+        amr_item<D, MODE, B, P, NT>(pa, w, L, n_shock, scnt);
     if ((tid & 63) == 0) {
         if (n_shock) atomicAdd(&scnt[0], n_shock);
-        if (n_fb) atomicAdd(&scnt[1], n_fb);
-        if (n_lim) atomicAdd(&scnt[2], n_lim);
     }
     __syncthreads();
     if (tid == 0) {
@@ -182,33 +166,18 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(EM_WAVES_PER
     }
 }
 
-// Adds a workgroup's counters to hierarchy `sc` (every thread calls it; the
-// n_* are reset).
-__device__ __forceinline__ void amr_flush_counters(DevScalars* sc, unsigned* scnt, unsigned& n_shock, unsigned& n_fb,
-                                                   unsigned& n_lim) {
+// Adds a workgroup's counters to hierarchy `sc` and clears them (every
+// thread calls it, after a barrier behind the last count).
+__device__ __forceinline__ void amr_flush_counters(DevScalars* sc, unsigned (&scnt)[3], unsigned& n_shock) {
     const int tid = threadIdx.x;
-#pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        n_shock += __shfl_xor(n_shock, off);
-        n_fb += __shfl_xor(n_fb, off);
-        n_lim += __shfl_xor(n_lim, off);
-    }
-    if (tid < 3) scnt[tid] = 0;
+    if ((tid & 63) == 0 && n_shock) atomicAdd(&scnt[0], n_shock);
     __syncthreads();
-    if ((tid & 63) == 0) {
-        if (n_shock) atomicAdd(&scnt[0], n_shock);
-        if (n_fb) atomicAdd(&scnt[1], n_fb);
-        if (n_lim) atomicAdd(&scnt[2], n_lim);
+    if (tid < 3) {
+        if (scnt[tid]) atomicAdd(&sc->counters[tid][blockIdx.x % kSlots][0], (unsigned long long)scnt[tid]);
+        scnt[tid] = 0;
     }
     __syncthreads();
-    if (tid == 0) {
-        const int slotc = blockIdx.x % kSlots;
-        if (scnt[0]) atomicAdd(&sc->counters[0][slotc][0], (unsigned long long)scnt[0]);
-        if (scnt[1]) atomicAdd(&sc->counters[1][slotc][0], (unsigned long long)scnt[1]);
-        if (scnt[2]) atomicAdd(&sc->counters[2][slotc][0], (unsigned long long)scnt[2]);
-    }
-    __syncthreads();
-    n_shock = n_fb = n_lim = 0;
+    n_shock = 0;
 }
 
 // The batched pass over the leaves of several hierarchies, whose blocks may
@@ -229,7 +198,9 @@ __global__ __launch_bounds__(kAmrMultiThreads) __attribute__((amdgpu_waves_per_e
         AmrLds<double, MODE, 32, 6> b32;
     } L;
     __shared__ unsigned int scnt[3];
-    unsigned int n_shock = 0, n_fb = 0, n_lim = 0;
+    unsigned int n_shock = 0;
+    if (threadIdx.x < 3) scnt[threadIdx.x] = 0;
+    __syncthreads();
     int cur = -1;
     for (long long w = blockIdx.x; w < m.total; w += gridDim.x) {
         int lo = 0, hi = m.n;
@@ -242,18 +213,18 @@ __global__ __launch_bounds__(kAmrMultiThreads) __attribute__((amdgpu_waves_per_e
         }
         const AmrPassArgs& pa = m.args[lo];  // read in place (global memory, cached)
         if (lo != cur) {
-            if (cur >= 0) amr_flush_counters(m.args[cur].a.sc, scnt, n_shock, n_fb, n_lim);
+            if (cur >= 0) amr_flush_counters(m.args[cur].a.sc, scnt, n_shock);
             cur = lo;
         }
         if (pa.a.sc->active == 0) continue;
         const long long wl = w - m.prefix[lo];
         switch (pa.a.bd[D]) {
-            case 8: amr_item<D, MODE, 8, 16, NT>(pa, wl, L.b8, n_shock, n_fb, n_lim); break;
-            case 16: amr_item<D, MODE, 16, 12, NT>(pa, wl, L.b16, n_shock, n_fb, n_lim); break;
-            default: amr_item<D, MODE, 32, 6, NT>(pa, wl, L.b32, n_shock, n_fb, n_lim); break;
+            case 8: amr_item<D, MODE, 8, 16, NT>(pa, wl, L.b8, n_shock, scnt); break;
+            case 16: amr_item<D, MODE, 16, 12, NT>(pa, wl, L.b16, n_shock, scnt); break;
+            default: amr_item<D, MODE, 32, 6, NT>(pa, wl, L.b32, n_shock, scnt); break;
         }
     }
-    if (cur >= 0) amr_flush_counters(m.args[cur].a.sc, scnt, n_shock, n_fb, n_lim);
+    if (cur >= 0) amr_flush_counters(m.args[cur].a.sc, scnt, n_shock);
 }
 
 template <int D, int MODE>

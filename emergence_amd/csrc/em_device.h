@@ -16,6 +16,7 @@
 #pragma once
 #include <hip/hip_runtime.h>
 
+#include <cmath>
 #include <cstdint>
 
 #include "em_div.h"
@@ -25,7 +26,10 @@ namespace em {
 template <class R>
 struct EosT {
     R gamma, p_inf, b, q;
-    R rg = R(1) / (gamma - R(1));  // correctly rounded reciprocal, for div_by
+    // 1 / (gamma - 1), correctly rounded, for div_by; NaN where the mid-range
+    // forms cannot vouch for their ranges (gamma near or below one, negative
+    // p_inf or q), which sends every operand the general way
+    R rg = gamma - R(1) >= R(1e-3) && gamma <= R(1e3) && p_inf >= R(0) && q >= R(0) ? R(1) / (gamma - R(1)) : R(NAN);
 };
 using Eos = EosT<double>;
 
@@ -128,10 +132,11 @@ __device__ __forceinline__ void to_prim_v(const EosT<R>& e, const R u[5], R w[5]
         w[1] = vx;
         w[2] = vy;
         w[3] = vz;
-        w[4] = (e.gamma - R(1.0)) * (en - e.q) / (v - e.b) - e.gamma * e.p_inf;
+        const R a = (e.gamma - R(1.0)) * (en - e.q), vb = v - e.b;
+        w[4] = div_by(a, vb, rcp_volume(e, rho, vb)) - e.gamma * e.p_inf;
         // an overflowing quotient leaves p infinite or NaN
-        if (!in_mid(rho) || too_small(u[1]) || too_small(u[2]) || too_small(u[3]) || too_small(u[4]) ||
-            !(fabs(w[4]) <= Mid<R>::huge)) {
+        if (!in_mid(rho) || !in_mid(vb) || too_small(u[1]) || too_small(u[2]) || too_small(u[3]) || too_small(u[4]) ||
+            too_small(a) || !(fabs(w[4]) <= Mid<R>::huge)) {
             to_prim(e, u, w);
             v = R(1.0) / rho;
         }
@@ -151,6 +156,12 @@ __device__ __forceinline__ R eos_rho_e_v(const EosT<R>& e, R rho, R p, R v) {
     }
 }
 
+// rcp_mid(vb) of vb = v - b, v = RN(1 / rho): without a covolume rho itself
+// is the reciprocal to an ulp and one Newton step finishes it
+__device__ __forceinline__ double rcp_volume(const Eos& e, double rho, double vb) {
+    return e.b == 0.0 ? rcp_step(vb, rho) : rcp_mid(vb);
+}
+
 // True where the conserved state q is admissible with so much room that the
 // rounded evaluation (to_prim, then admissible) cannot decide otherwise, and
 // is finite; no division.  With d = (E - |m|^2 / 2 rho - rho q - p_inf (1 -
@@ -166,14 +177,16 @@ __device__ __forceinline__ bool clearly_admissible(const EosT<R>& e, const R q[5
     const R d = a - k - y - z;
     const R size = fabs(a) + k + fabs(y) + fabs(z);
     return in_mid(rho) && fabs(rb) <= R(0.5) && d > Mid<R>::margin * size && d > Mid<R>::lo * Mid<R>::lo &&
-           size < Mid<R>::hi * Mid<R>::hi && e.rg > R(0.0) && e.rg < R(100.0);
+           size < Mid<R>::hi * Mid<R>::hi && e.gamma - R(1.0) > R(0.01);
 }
 
 // The flux and the selected star state of HLLC once the two sound speeds
-// and conserved states are known (system.rs:268-312).
-template <int D, class R>
+// and conserved states are known (system.rs:268-312).  MID: densities, sound
+// speeds and velocities are in the middle of the exponent range, il and ir
+// their densities' reciprocals (rcp_mid).
+template <int D, bool MID = false, class R>
 __device__ __forceinline__ void hllc_flux(const R wl[5], const R wr[5], const R ql[5], const R qr[5], R cl, R cr,
-                                          R f[5]) {
+                                          R il, R ir, R f[5]) {
     constexpr int un = 1 + D;
     R ul = wl[un], ur = wr[un];
     R sl = fmin(ul - cl, ur - cr);
@@ -199,14 +212,20 @@ __device__ __forceinline__ void hllc_flux(const R wl[5], const R wr[5], const R 
     }
     R s = left ? sl : sr;
     R rho = w[0], u = w[un];
-    R fac = rho * (s - u) / (s - ss);
+    const R h = rho * (s - u);
+    R fac = h / (s - ss);
+    R en;
+    if constexpr (MID)
+        en = div_by(q[4], rho, left ? il : ir);
+    else
+        en = q[4] / rho;
     R qs[5];
     qs[0] = fac;
     qs[1] = fac * w[1];
     qs[2] = fac * w[2];
     qs[3] = fac * w[3];
     qs[un] = fac * ss;
-    qs[4] = fac * (q[4] / rho + (ss - u) * (ss + w[4] / (rho * (s - u))));
+    qs[4] = fac * (en + (ss - u) * (ss + w[4] / h));
     R fw[5];
     phys_flux<D>(w, q, fw);
 #pragma unroll
@@ -220,7 +239,7 @@ __device__ __forceinline__ void hllc(const EosT<R>& e, const R wl[5], const R wr
     R ql[5], qr[5];
     to_cons(e, wl, ql);
     to_cons(e, wr, qr);
-    hllc_flux<D>(wl, wr, ql, qr, cl, cr, f);
+    hllc_flux<D>(wl, wr, ql, qr, cl, cr, cl, cr, f);
 }
 
 // KEEP-PE two-point flux: system.rs:317-334
@@ -289,19 +308,20 @@ __device__ __forceinline__ R weno5z_interp(R v0, R v1, R v2, R v3, R v4) {
 }
 
 // WCNS midpoint flux: characteristic WENO5-Z interpolation of the six
-// primitive states s[0..5] = w_{j-2..j+3} to the midpoint j+1/2, first-order
-// fallback on an inadmissible state, HLLC there.  scheme.rs:286-333, with the
-// eigenvectors of system.rs:232-258 applied in sparse form.
-// Returns true on the first-order fallback.
-template <int D, class R>
-__device__ __forceinline__ bool midpoint_flux(const EosT<R>& e, const R (&s)[6][5], R f[5]) {
+// primitive states w_{j-2..j+3}, component k of cell j read through ld(j, k),
+// to the midpoint j+1/2, first-order fallback on an inadmissible state, HLLC
+// there.  scheme.rs:286-333, with the eigenvectors of system.rs:232-258
+// applied in sparse form.  Returns true on the first-order fallback.
+// FIELDS: the characteristic fields in a loop of one body (for FP64, where
+// midpoint_flux_mid takes almost every midpoint and this is cold code that
+// only fills the instruction cache), else unrolled.
+template <int D, bool FIELDS, class R, class LD>
+__device__ __forceinline__ bool midpoint_flux(const EosT<R>& e, LD&& ld, R f[5]) {
     constexpr int un = 1 + D;
     constexpr int t1 = 1 + (D + 1) % 3;
     constexpr int t2 = 1 + (D + 2) % 3;
-    R rho = R(0.5) * (s[2][0] + s[3][0]);
-    R avun = R(0.5) * (s[2][un] + s[3][un]);
-    R avp = R(0.5) * (s[2][4] + s[3][4]);
-    (void)avun;
+    R rho = R(0.5) * (ld(2, 0) + ld(3, 0));
+    R avp = R(0.5) * (ld(2, 4) + ld(3, 4));
     R c = sound_speed(e, rho, avp);
     // L rows (waves u-c, entropy, shear t1, shear t2, u+c)
     R l0un = -rho / (R(2.0) * c);
@@ -309,46 +329,84 @@ __device__ __forceinline__ bool midpoint_flux(const EosT<R>& e, const R (&s)[6][
     R l14 = -R(1.0) / (c * c);
     R l4un = rho / (R(2.0) * c);
     R l44 = R(1.0) / (R(2.0) * c * c);
-    R ch[6][5];
-#pragma unroll
-    for (int k = 0; k < 6; ++k) {
-        ch[k][0] = l0un * s[k][un] + l04 * s[k][4];
-        ch[k][1] = s[k][0] + l14 * s[k][4];
-        ch[k][2] = s[k][t1];
-        ch[k][3] = s[k][t2];
-        ch[k][4] = l4un * s[k][un] + l44 * s[k][4];
-    }
-    R cl[5], cr[5];
-#pragma unroll
-    for (int a = 0; a < 5; ++a) {
-        cl[a] = weno5z_interp(ch[0][a], ch[1][a], ch[2][a], ch[3][a], ch[4][a]);
-        cr[a] = weno5z_interp(ch[5][a], ch[4][a], ch[3][a], ch[2][a], ch[1][a]);
-    }
     // R columns: r[0][0]=r[0][1]=r[0][4]=1, r[un][0]=-c/rho, r[un][4]=c/rho,
     // r[t1][2]=r[t2][3]=1, r[4][0]=r[4][4]=c*c
     R run0 = -c / rho, run4 = c / rho, r40 = c * c;
     R wl[5], wr[5];
-    wl[0] = cl[0] + cl[1] + cl[4];
-    wr[0] = cr[0] + cr[1] + cr[4];
-    wl[un] = run0 * cl[0] + run4 * cl[4];
-    wr[un] = run0 * cr[0] + run4 * cr[4];
-    wl[t1] = cl[2];
-    wr[t1] = cr[2];
-    wl[t2] = cl[3];
-    wr[t2] = cr[3];
-    wl[4] = r40 * cl[0] + r40 * cl[4];
-    wr[4] = r40 * cr[0] + r40 * cr[4];
+#pragma unroll
+    for (int k = 0; k < 5; ++k) wl[k] = wr[k] = R(0.0);
+    auto field = [&](int a) {
+        R ch[6];
+        if (a == 0) {
+#pragma unroll
+            for (int j = 0; j < 6; ++j) ch[j] = l0un * ld(j, un) + l04 * ld(j, 4);
+        } else if (a == 1) {
+#pragma unroll
+            for (int j = 0; j < 6; ++j) ch[j] = ld(j, 0) + l14 * ld(j, 4);
+        } else if (a == 4) {
+#pragma unroll
+            for (int j = 0; j < 6; ++j) ch[j] = l4un * ld(j, un) + l44 * ld(j, 4);
+        } else if (a == 2) {
+#pragma unroll
+            for (int j = 0; j < 6; ++j) ch[j] = ld(j, t1);
+        } else {
+#pragma unroll
+            for (int j = 0; j < 6; ++j) ch[j] = ld(j, t2);
+        }
+        const R cl = weno5z_interp(ch[0], ch[1], ch[2], ch[3], ch[4]);
+        const R cr = weno5z_interp(ch[5], ch[4], ch[3], ch[2], ch[1]);
+        if (a == 0) {
+            wl[0] = cl;
+            wr[0] = cr;
+            wl[un] = run0 * cl;
+            wr[un] = run0 * cr;
+            wl[4] = r40 * cl;
+            wr[4] = r40 * cr;
+        } else if (a == 1) {
+            wl[0] = wl[0] + cl;
+            wr[0] = wr[0] + cr;
+        } else if (a == 2) {
+            wl[t1] = cl;
+            wr[t1] = cr;
+        } else if (a == 3) {
+            wl[t2] = cl;
+            wr[t2] = cr;
+        } else {
+            wl[0] = wl[0] + cl;
+            wr[0] = wr[0] + cr;
+            wl[un] = wl[un] + run4 * cl;
+            wr[un] = wr[un] + run4 * cr;
+            wl[4] = wl[4] + r40 * cl;
+            wr[4] = wr[4] + r40 * cr;
+        }
+    };
+    if constexpr (FIELDS) {
+#pragma unroll 1
+        for (int a = 0; a < 5; ++a) field(a);
+    } else {
+#pragma unroll
+        for (int a = 0; a < 5; ++a) field(a);
+    }
     bool fb = false;
     if (!admissible(e, wl[0], wl[4]) || !admissible(e, wr[0], wr[4])) {
         fb = true;
 #pragma unroll
         for (int k = 0; k < 5; ++k) {
-            wl[k] = s[2][k];
-            wr[k] = s[3][k];
+            wl[k] = ld(2, k);
+            wr[k] = ld(3, k);
         }
     }
     hllc<D>(e, wl, wr, f);
     return fb;
+}
+
+// weno5z_interp where every |v| < 2^-200: beta + eps is eps and 1 + r^2 is 1,
+// which leaves the linear weights, whose sum is 1.
+__device__ __forceinline__ double weno5_linear(double v0, double v1, double v2, double v3, double v4) {
+    const double q0 = (3.0 * v0 - 10.0 * v1 + 15.0 * v2) * 0.125;
+    const double q1 = (-v1 + 6.0 * v2 + 3.0 * v3) * 0.125;
+    const double q2 = (3.0 * v2 + 6.0 * v3 - v4) * 0.125;
+    return 0.0625 * q0 + 0.625 * q1 + 0.3125 * q2;
 }
 
 // Both WENO5-Z interpolations of a midpoint's six point values, left (v0..v4)
@@ -364,10 +422,15 @@ __device__ __forceinline__ bool midpoint_flux(const EosT<R>& e, const R (&s)[6][
 //   * tau / (beta + eps): the reciprocals of the three (rcp3_mid), and of the
 //     two weight sums (rcp2_mid), are taken jointly.  A tau too small for the
 //     core leaves 1 + r^2 = 1 either way.
-// top is raised to the largest beta's high word, ok cleared where the last
+// left and right are 8 times the interpolated values.  top is raised to the
+// high word of the product of the three beta + eps, ok cleared where the last
 // quotient needs the general division: the caller falls back to
-// weno5z_interp unless ok and top below beta_max.  95 issue slots a side (a
-// reciprocal counts four) against about 125.
+// weno5z_interp unless ok and top below beta_max.  TINY: zero fields and
+// fields below 2^-200 are taken here as well (ahead of a front in gas at
+// rest the velocities fall off to denormals over many cells: a tenth of all
+// cells in a shock-bubble run).  91 issue slots a side (a reciprocal counts
+// four) against about 125.
+template <bool TINY>
 __device__ __forceinline__ void weno5z_pair(const double v[6], double& left, double& right, unsigned& top, bool& ok) {
 #ifndef EM_CONTRACT
     const double m0 = 3.0 * v[0], m2 = 3.0 * v[2], m3 = 3.0 * v[3], m5 = 3.0 * v[5];
@@ -402,9 +465,8 @@ __device__ __forceinline__ void weno5z_pair(const double v[6], double& left, dou
 #endif
         const double tau = fabs(b0 - b2);
         const double d0 = b0 + 1e-40, d1 = b1 + 1e-40, d2 = b2 + 1e-40;
-        top = max(max(top, top_word(d0)), max(top_word(d1), top_word(d2)));
         double i0, i1, i2;
-        rcp3_mid(d0, d1, d2, i0, i1, i2);
+        top = max(top, top_word(rcp3_mid(d0, d1, d2, i0, i1, i2)));
         const double r0 = div_by(tau, d0, i0), r1 = div_by(tau, d1, i1), r2 = div_by(tau, d2, i2);
         const double a0 = 1.0 + r0 * r0;
         const double a1 = 10.0 * (1.0 + r1 * r1);
@@ -414,10 +476,19 @@ __device__ __forceinline__ void weno5z_pair(const double v[6], double& left, dou
     }
     double il, ir;
     rcp2_mid(S[0], S[1], il, ir);
-    const double ql = div_by_fix(N[0], S[0], il), qr = div_by_fix(N[1], S[1], ir);
-    ok = ok && (fabs(ql) >= Mid<double>::tiny || N[0] == 0.0) && (fabs(qr) >= Mid<double>::tiny || N[1] == 0.0);
-    left = 0.125 * ql;
-    right = 0.125 * qr;
+    left = div_by_fix(N[0], S[0], il);
+    right = div_by_fix(N[1], S[1], ir);
+    bool fine = fabs(left) >= Mid<double>::tiny && fabs(right) >= Mid<double>::tiny;
+    if (TINY && !fine) {
+        fine = (fabs(left) >= Mid<double>::tiny || N[0] == 0.0) && (fabs(right) >= Mid<double>::tiny || N[1] == 0.0);
+        const double m = fmax(fmax(fmax(fabs(v[0]), fabs(v[1])), fmax(fabs(v[2]), fabs(v[3]))), fmax(fabs(v[4]), fabs(v[5])));
+        if (!fine && m < 0x1p-200) {
+            fine = true;
+            left = 8.0 * weno5_linear(v[0], v[1], v[2], v[3], v[4]);
+            right = 8.0 * weno5_linear(v[5], v[4], v[3], v[2], v[1]);
+        }
+    }
+    ok = ok && fine;
 }
 
 // midpoint_flux for operands in the middle of the exponent range, stencil
@@ -444,23 +515,25 @@ __device__ __forceinline__ bool midpoint_flux_mid(const Eos& e, bool zero1, bool
     const double irho = rcp_mid(rho);
     const double v = inv_by(rho, irho);
     const double vb = v - e.b;
-    const double c2 = div_by(e.gamma * (avp + e.p_inf) * v * v, vb, rcp_mid(vb));
-    bool ok = in_mid(rho) && in_mid(vb) && in_mid(c2) && e.rg > 0.0 && e.rg <= Mid<double>::hi;
-    const double c = sqrt_mid(c2);
+    const double c2 = div_by(e.gamma * (avp + e.p_inf) * v * v, vb, rcp_volume(e, rho, vb));
+    double ic;
+    const double c = sqrt_mid(c2, ic);
     const double cc = c * c;
-    const double lu = 0.5 * div_by(rho, c, rcp_mid(c));  // rho / (2 c)
-    const double lp = 0.5 * inv_by(cc, rcp_mid(cc));     // 1 / (2 c^2)
-    const double ru = div_by(c, rho, irho);                 // c / rho
+    const double lu = 0.5 * div_by(rho, c, ic);                  // rho / (2 c)
+    const double lp = 0.5 * inv_by(cc, rcp_step(cc, ic * ic));   // 1 / (2 c^2)
+    const double ru = 0.125 * div_by(c, rho, irho);              // c / rho, of the sums times 8
+    const double cc8 = 0.125 * cc;
+    bool ok = e.rg > 0.0;
     unsigned top = 0;
     double wl[5], wr[5];
     {
         double ch[6], l0, r0, l1, r1, l4, r4;
 #pragma unroll
         for (int j = 0; j < 6; ++j) ch[j] = lp * ld(j, 4) - lu * ld(j, un);
-        weno5z_pair(ch, l0, r0, top, ok);
+        weno5z_pair<false>(ch, l0, r0, top, ok);
 #pragma unroll
         for (int j = 0; j < 6; ++j) ch[j] = lp * ld(j, 4) + lu * ld(j, un);
-        weno5z_pair(ch, l4, r4, top, ok);
+        weno5z_pair<false>(ch, l4, r4, top, ok);
 #pragma unroll
         for (int j = 0; j < 6; ++j)
 #ifndef EM_CONTRACT
@@ -468,13 +541,13 @@ __device__ __forceinline__ bool midpoint_flux_mid(const Eos& e, bool zero1, bool
 #else
             ch[j] = ld(j, 0) - 2.0 * lp * ld(j, 4);
 #endif
-        weno5z_pair(ch, l1, r1, top, ok);
-        wl[0] = l0 + l1 + l4;
-        wr[0] = r0 + r1 + r4;
+        weno5z_pair<false>(ch, l1, r1, top, ok);
+        wl[0] = 0.125 * (l0 + l1 + l4);
+        wr[0] = 0.125 * (r0 + r1 + r4);
         wl[un] = ru * l4 - ru * l0;
         wr[un] = ru * r4 - ru * r0;
-        wl[4] = cc * l0 + cc * l4;
-        wr[4] = cc * r0 + cc * r4;
+        wl[4] = cc8 * l0 + cc8 * l4;
+        wr[4] = cc8 * r0 + cc8 * r4;
     }
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -484,16 +557,25 @@ __device__ __forceinline__ bool midpoint_flux_mid(const Eos& e, bool zero1, bool
         for (int j = 0; j < 6; ++j) ch[j] = ld(j, t);
         wl[t] = wr[t] = 0.0;
         if (!(s ? zero2 : zero1) || __any(any_bits(ch[0], ch[1], ch[2]) | any_bits(ch[3], ch[4], ch[5])))
-            weno5z_pair(ch, wl[t], wr[t], top, ok);
+            weno5z_pair<true>(ch, wl[t], wr[t], top, ok);
+        wl[t] *= 0.125;
+        wr[t] *= 0.125;
     }
     // both states admissible, with sound speeds in range
     const double il = rcp_mid(wl[0]), ir = rcp_mid(wr[0]);
     const double vl = inv_by(wl[0], il), vr = inv_by(wr[0], ir);
     const double vbl = vl - e.b, vbr = vr - e.b;
-    const double c2l = div_by(e.gamma * (wl[4] + e.p_inf) * vl * vl, vbl, rcp_mid(vbl));
-    const double c2r = div_by(e.gamma * (wr[4] + e.p_inf) * vr * vr, vbr, rcp_mid(vbr));
-    ok = ok && top < top_word(Mid<double>::beta_max) && in_mid(wl[0]) && in_mid(wr[0]) && in_mid(vbl) && in_mid(vbr) &&
-         in_mid(c2l) && in_mid(c2r) && wl[4] + e.p_inf > 0.0 && wr[4] + e.p_inf > 0.0;
+    const double c2l = div_by(e.gamma * (wl[4] + e.p_inf) * vl * vl, vbl, rcp_volume(e, wl[0], vbl));
+    const double c2r = div_by(e.gamma * (wr[4] + e.p_inf) * vr * vr, vbr, rcp_volume(e, wr[0], vbr));
+    // all of [lo, hi]: high words order like positive values, a negative one
+    // or NaN is above them all
+    const unsigned mn = min(min(min(top_word(rho), top_word(vb)), min(top_word(c2), top_word(wl[0]))),
+                            min(min(min(top_word(wr[0]), top_word(vbl)), top_word(vbr)), min(top_word(c2l), top_word(c2r))));
+    const unsigned mx = max(max(max(top_word(rho), top_word(vb)), max(top_word(c2), top_word(wl[0]))),
+                            max(max(max(top_word(wr[0]), top_word(vbl)), top_word(vbr)), max(top_word(c2l), top_word(c2r))));
+    ok = ok && top < top_word(Mid<double>::beta_max) && mn >= top_word(Mid<double>::lo) &&
+         mx < top_word(Mid<double>::hi) && fmax(fabs(wl[un]), fabs(wr[un])) < Mid<double>::hi;
+    if (!ok) return false;
     double ql[5], qr[5];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -505,11 +587,10 @@ __device__ __forceinline__ bool midpoint_flux_mid(const Eos& e, bool zero1, bool
         q[2] = w[0] * w[2];
         q[3] = w[0] * w[3];
         const double a = (w[4] + e.gamma * e.p_inf) * (s ? vbr : vbl);
-        ok = ok && !too_small(a);
         q[4] = w[0] * (div_by(a, e.gamma - 1.0, e.rg) + e.q) + ke;
     }
-    if (!ok) return false;
-    hllc_flux<D>(wl, wr, ql, qr, sqrt_mid(c2l), sqrt_mid(c2r), f);
+    double x;
+    hllc_flux<D, true>(wl, wr, ql, qr, sqrt_mid(c2l, x), sqrt_mid(c2r, x), il, ir, f);
     return true;
 }
 
@@ -611,7 +692,7 @@ __device__ __forceinline__ void bc_ghost(const EosT<R>& e, int n, int g, const i
             break;
         }
         const int side = x >= n ? 1 : 0;
-        const int k = kind[side];
+        const int k = side ? kind[1] : kind[0];
         if (k == 2) {
             x = side == 0 ? -1 - x : 2 * n - 1 - x;
             flip = !flip;
@@ -623,12 +704,15 @@ __device__ __forceinline__ void bc_ghost(const EosT<R>& e, int n, int g, const i
             ld(side == 0 ? 0 : n - 1, u);
         } else if (k == 3) {
 #pragma unroll
-            for (int q = 0; q < 5; ++q) u[q] = state[side][q];
+            for (int q = 0; q < 5; ++q) u[q] = side ? state[1][q] : state[0][q];
         } else {
             R ub[5], ub1[5];
             ld(side == 0 ? 0 : n - 1, ub);
             ld(side == 0 ? 1 : n - 2, ub1);
-            characteristic_ghost<D>(e, ub, ub1, state[side], side, side == 0 ? R(-x) : R(x - n + 1), u);
+            R uf[5];
+#pragma unroll
+            for (int q = 0; q < 5; ++q) uf[q] = side ? state[1][q] : state[0][q];
+            characteristic_ghost<D>(e, ub, ub1, uf, side, side == 0 ? R(-x) : R(x - n + 1), u);
         }
         break;
     }

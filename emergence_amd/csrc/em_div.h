@@ -22,9 +22,9 @@ struct Mid;
 template <>
 struct Mid<double> {
     static constexpr double lo = 0x1p-100, hi = 0x1p+100;  // densities, squared sound speeds
-    static constexpr double tiny = 0x1p-400;               // quotients and dividends below go the general way
+    static constexpr double tiny = 0x1p-900;               // quotients and dividends below go the general way
     static constexpr double huge = 0x1p+800;
-    static constexpr double beta_max = 0x1p+100;  // WENO smoothness indicators: products of three stay normal
+    static constexpr double beta_max = 0x1p+100;  // product of three WENO smoothness indicators
     static constexpr double margin = 1e-9;        // relative slack of clearly_admissible (rounding: about 1e-15)
 };
 template <>
@@ -69,27 +69,31 @@ __device__ __forceinline__ double inv_by(double b, double r) { return rcp_step(b
 
 // sqrt(x), x within [lo, hi]: v_rsq and the coupled Newton iteration of
 // sqrt and 1 / (2 sqrt) with two residual corrections (Goldschmidt; Markstein
-// 2000), correctly rounded
-__device__ __forceinline__ double sqrt_mid(double x) {
+// 2000), correctly rounded; inv = rcp_mid of the root, from the iteration's
+// own 1 / (2 sqrt).
+__device__ __forceinline__ double sqrt_mid(double x, double& inv) {
     const double y = __builtin_amdgcn_rsq(x);
     double g = x * y, h = 0.5 * y;
     const double r = __builtin_fma(-h, g, 0.5);
     g = __builtin_fma(g, r, g);
     h = __builtin_fma(h, r, h);
     g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
-    return __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    g = __builtin_fma(__builtin_fma(-g, g, x), h, g);
+    inv = rcp_step(g, h + h);
+    return g;
 }
 
-// 1/d0, 1/d1, 1/d2 through one reciprocal of the product (doubles of
-// [2^-133, 2^100]: the products stay within 2^+-400); each gets its own last
-// Newton step.  Singly 8 issue slots each, jointly 18 for the three.
-__device__ __forceinline__ void rcp3_mid(double d0, double d1, double d2, double& r0, double& r1, double& r2) {
+// 1/d0, 1/d1, 1/d2 through one reciprocal of the product, which is returned
+// (doubles of at least 2^-133 with a product up to 2^100); each gets its own
+// last Newton step.  Singly 8 issue slots each, jointly 18 for the three.
+__device__ __forceinline__ double rcp3_mid(double d0, double d1, double d2, double& r0, double& r1, double& r2) {
     const double p = d0 * d1, pp = p * d2;
     const double r = rcp_step(pp, __builtin_amdgcn_rcp(pp));
     const double r01 = r * d2;
     r0 = rcp_step(d0, r01 * d1);
     r1 = rcp_step(d1, r01 * d0);
     r2 = rcp_step(d2, r * p);
+    return pp;
 }
 // the same for two doubles of [2^-1, 2^480]
 __device__ __forceinline__ void rcp2_mid(double d0, double d1, double& r0, double& r1) {
@@ -102,6 +106,34 @@ __device__ __forceinline__ void rcp2_mid(double d0, double d1, double& r0, doubl
 // High word of a non-negative value, which orders like the value (NaN above
 // all): a running bound at one instruction per two values.
 __device__ __forceinline__ unsigned top_word(double x) { return (unsigned)__double2hiint(x); }
+
+// a value equal on all lanes, kept in scalar registers
+__device__ __forceinline__ double wave_uniform(double x) {
+    return __hiloint2double(__builtin_amdgcn_readfirstlane(__double2hiint(x)),
+                            __builtin_amdgcn_readfirstlane(__double2loint(x)));
+}
+
+// Scalar-cache copy of *p, the same for the whole wave, from memory that no
+// kernel running meanwhile writes.  Through an ordinary pointer a kernel that
+// also stores reads such arguments with vector loads into vector registers.
+template <class T>
+__device__ __forceinline__ T scalar_copy(const T* p) {
+    static_assert(sizeof(T) % 4 == 0, "whole words");
+    const __attribute__((address_space(4))) unsigned* s =
+        (const __attribute__((address_space(4))) unsigned*)(unsigned long long)p;
+    unsigned t[sizeof(T) / 4];
+#pragma unroll
+    for (int i = 0; i < (int)(sizeof(T) / 4); ++i) t[i] = s[i];
+    T r;
+    __builtin_memcpy(&r, t, sizeof(T));
+    return r;
+}
+
+// x, unknown to the optimiser
+__device__ __forceinline__ int opaque(int x) {
+    asm volatile("" : "+v"(x));
+    return x;
+}
 
 // some bit of the three set (false only for +0, +0, +0)
 __device__ __forceinline__ unsigned any_bits(double a, double b, double c) {

@@ -7,12 +7,12 @@
 
 namespace em {
 
-// Tile shapes (cells along the axis x pencils, threads); index = cfg id.
-// Shapes 4..9 give exactly one midpoint per thread ((T+5)*P == NT); shape 9
-// puts 16 pencils in a workgroup, so that a strided pass reads whole 128-byte
-// lines (16 neighbouring cells of the innermost axis).
-constexpr TileCfg kTileCfgs[] = {{32, 16, 640}, {64, 8, 576}, {128, 4, 576}, {256, 2, 576}, {27, 8, 256},
-                                 {59, 4, 256},  {59, 8, 512}, {27, 16, 512}, {123, 4, 512}, {59, 16, 1024}};
+// Tile shapes (cells along the axis x pencils, threads); index = cfg id.  A
+// strided pass reads P neighbouring cells of the innermost axis.  One thread
+// per cell (T P == NT) suits segments of many tiles, one per midpoint
+// ((T + 5) P == NT) those of one tile.
+constexpr TileCfg kTileCfgs[] = {{32, 8, 256}, {16, 16, 256}, {64, 8, 512}, {27, 8, 256}, {59, 4, 256},
+                                 {27, 4, 128}, {27, 2, 64}, {59, 1, 64}, {16, 4, 64}, {123, 4, 512}};
 constexpr int kNumTileCfgs = 10;
 
 #define EM_DECLARE_LAUNCHERS                                                               \

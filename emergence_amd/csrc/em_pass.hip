@@ -78,162 +78,175 @@ __device__ __forceinline__ void ghost_state(const PassArgsT<Real>& a, long long 
     bc_ghost<D>(a.eos, a.n[D], g, a.bc_kind, a.bc_state, ld, u);
 }
 
-// LDS of one tile (declared by the kernels, passed to axis_tile)
-template <class Real, int MODE, int T, int P, int NT>
-struct TileLds {
-    static constexpr bool HYB = MODE == MODE_HYBRID;
-    Real sw[5][T + 10][P];
-    Real sre[T + 10][P];  // rho_e of each cell
-    Real sm[5][T + 5][P];
-    Real ss[2][HYB ? T + 10 : 1][P];
-    Real sth[HYB ? T + 1 : 1][P];
+// LDS of a pass (declared by the kernels, passed to axis_segment)
+template <class Real, int MODE, int T, int P, bool CF, int NT>
+struct PassLds : Tile<Real, MODE, T, P, CF> {
     double sred[NT / 64 + 1];  // per-wave CFL rate (in double for the slot max)
     unsigned int scnt[3];
 };
 
-// Tile `bid` of one axis pass described by `a` (every thread of the
+// Segment `bid` of one axis pass described by `a`: a.seg cells of P
+// neighbouring pencils, walked in tiles of T cells (every thread of the
 // workgroup calls it; it returns uniformly).
-template <class Real, int D, int MODE, int T, int P, int NT>
-__device__ __forceinline__ void axis_tile(const PassArgsT<Real>& a, int bid, TileLds<Real, MODE, T, P, NT>& L) {
-    constexpr int C = T + 10;  // cells held in LDS
+template <class Real, int D, int MODE, int T, int P, bool CF, int NT>
+__device__ __forceinline__ void axis_segment(const PassArgsT<Real>& a, int bid, PassLds<Real, MODE, T, P, CF, NT>& L) {
+    using TL = Tile<Real, MODE, T, P, CF>;
     constexpr bool HYB = MODE == MODE_HYBRID;
     auto& sw = L.sw;
-    auto& sre = L.sre;
     auto& sm = L.sm;
-    auto& ss = L.ss;
-    auto& sth = L.sth;
     auto& sred = L.sred;
     auto& scnt = L.scnt;
 
-    if (a.sc->active == 0) return;
     const int tid = threadIdx.x;
-    const int tile = bid % a.ntile;
-    const int rest = bid / a.ntile;
+    const int sg = bid % a.nseg;
+    const int rest = bid / a.nseg;
     const int gF = rest % a.ngroup;
     const int sI = rest / a.ngroup;
     const int nD = a.n[D];
-    const int nF = a.n[a.fast_axis];
-    const int c0 = tile * T;
-    const int Tv = min(T, nD - c0);
+    const int nF = a.n_fast;
+    const int s0 = sg * a.seg, s1 = min(s0 + a.seg, nD);
     const int p0 = gF * P;
     const int Pv = min(P, nF - p0);
     const long long sD = a.stride[D];
-    const long long sF = a.stride[a.fast_axis];
-    const long long base = (long long)sI * a.stride[a.slow_axis] + (long long)p0 * sF;
+    const long long sF = a.s_fast;
+    const long long base = (long long)sI * a.s_slow + (long long)p0 * sF;
     const long long nc = a.ncell;
     const EosT<Real> e = a.eos;
     if (tid < 3) scnt[tid] = 0;
-
-    // ---- 1. load + primitives
-    for (int it = tid; it < C * P; it += NT) {
-        int c, p;
-        if (a.dfast) {
-            c = it % C;
-            p = it / C;
-        } else {
-            p = it % P;
-            c = it / P;
-        }
-        if (p >= Pv || c >= Tv + 10) continue;
-        const int g = c0 - 5 + c;
-        const long long pen = base + (long long)p * sF;
-        Real u[5], w[5];
-        if (g >= 0 && g < nD) {
-            const long long idx = pen + (long long)g * sD;
-#pragma unroll
-            for (int k = 0; k < 5; ++k) u[k] = a.U[k * nc + idx];
-        } else {
-            ghost_state<D>(a, pen, g, u);
-        }
-        Real v;
-        to_prim_v(e, u, w, v);
-#pragma unroll
-        for (int k = 0; k < 5; ++k) sw[k][c][p] = w[k];
-        sre[c][p] = eos_rho_e_v(e, w[0], w[4], v);
-        if constexpr (HYB) {
-            // Euler::sensor, system.rs:409-413
-            ss[0][c][p] = log(fmax(w[0], Real(1e-300)));
-            ss[1][c][p] = log(fmax(w[4] + e.p_inf, Real(1e-300)));
-        }
-    }
-    __syncthreads();
-
-    unsigned int n_shock = 0, n_fb = 0, n_lim = 0;
-    double lam = 0.0;
-    if (a.ndim_pos > 0.0) {
-        const double dt = a.stage_dt_host ? a.stage_dt : a.sc->dt;
-        lam = a.ndim_pos * dt / a.dx_d;  // solver.rs:393
-    }
-    tile_faces<D, MODE, T, P, NT>(sw, sre, sm, ss, sth, Tv, Pv, c0, nD, e, Real(lam), a.tol,
-                                 !a.active[(D + 1) % 3], !a.active[(D + 2) % 3], n_shock, n_fb, n_lim);
-
-    // ---- 5. divergence, fused RK stage and CFL rate
+    // read together and tested behind the first tile's loads: one round trip
+    const int active = a.sc->active;
+    const double dt_d = wave_uniform(a.sc->dt);
+    double lam_d = 0.0;
+    if (a.ndim_pos > 0.0) lam_d = a.ndim_pos * (a.stage_dt_host ? a.stage_dt : dt_d) / a.dx_d;  // solver.rs:393
+    const Real lam = Real(wave_uniform(lam_d));
+    const Real dt = Real(dt_d);
+    unsigned int n_shock = 0;
     double rate = 0.0;
-    const Real dt = Real(a.sc->dt);
-    for (int it = tid; it < T * P; it += NT) {
+
+#pragma unroll 1
+    for (int c0 = s0; c0 < s1; c0 += T) {
+        // opaque in every turn: addresses are formed where they are used
+        // (hoisted out of the loop they fill the registers and spill)
+        const int tid = opaque(threadIdx.x);
+        const bool first = HYB || c0 == s0;
+        const int Tv = min(T, s1 - c0);
+        // ---- 1. load + primitives
+#pragma unroll 1
+        for (int it = tid - (first ? TL::HC * P : 0); it < T * P; it += NT) {
+            int c, p;
+            TL::template item<TL::HC>(it, c, p);
+            const int g = c0 - 5 + c;
+            if (p >= Pv || c >= Tv + TL::HC || g >= nD + 5) continue;
+            const long long pen = base + (long long)p * sF;
+            Real u[5], w[5];
+            if (g >= 0 && g < nD) {
+                const long long idx = pen + (long long)g * sD;
+#pragma unroll
+                for (int k = 0; k < 5; ++k) u[k] = a.U[k * nc + idx];
+            } else {
+                ghost_state<D>(a, pen, g, u);
+            }
+            Real v;
+            to_prim_v(e, u, w, v);
+            const int q = TL::at(c, p);
+#pragma unroll
+            for (int k = 0; k < 5; ++k) sw[k][q] = w[k];
+            L.sre[q] = eos_rho_e_v(e, w[0], w[4], v);
+            if constexpr (HYB) {
+                // Euler::sensor, system.rs:409-413
+                L.ss[0][q] = log(fmax(w[0], Real(1e-300)));
+                L.ss[1][q] = log(fmax(w[4] + e.p_inf, Real(1e-300)));
+            }
+        }
+        if (active == 0) return;
+        // the midpoints and the face flux taken over from the last tile
+        if (!first) {
+            if (tid < TL::HM * P) {
+                const int m = CF ? tid % TL::HM : tid / P, p = CF ? tid / TL::HM : tid % P;
+#pragma unroll
+                for (int k = 0; k < 5; ++k) {
+                    const Real x = sm[k][TL::mt(T + m, p)];
+                    if (m == 0) L.sf[k][p] = sm[k][TL::mt(T - 1, p)];
+                    sm[k][TL::mt(m, p)] = x;
+                }
+            }
+        }
+        __syncthreads();
+
         int c, p;
-        if (a.dfast) {
-            c = it % T;
-            p = it / T;
-        } else {
-            p = it % P;
-            c = it / P;
-        }
-        if (p >= Pv || c >= Tv) continue;
+        TL::template item<0>(tid, c, p);
+        const bool mine = tid < T * P && p < Pv && c < Tv;
         const long long idx = base + (long long)p * sF + (long long)(c0 + c) * sD;
-        Real r[5];
+        Real r[5], u0[5], us[5];
+        tile_faces<D, MODE, NT>(L, tid, first, Tv, Pv, c0, s0, s1, nD, e, lam, a.tol, !a.active[(D + 1) % 3],
+                                !a.active[(D + 2) % 3], n_shock, scnt, [&] {
 #pragma unroll
-        for (int k = 0; k < 5; ++k) {
-            const Real prev = a.first ? Real(0.0) : a.R[k * nc + idx];
-            r[k] = prev - (sm[k][c + 1][p] - sm[k][c][p]) * a.inv_dx;
-        }
-        if (a.rk_stage == 0) {
-#pragma unroll
-            for (int k = 0; k < 5; ++k) a.R[k * nc + idx] = r[k];
-        } else {
-            Real un_[5];
+                                    for (int k = 0; k < 5; ++k) {
+                                        r[k] = a.first || !mine ? Real(0.0) : a.R[k * nc + idx];
+                                        u0[k] = a.rk_stage == 0 || !mine ? Real(0.0) : a.U0[k * nc + idx];
+                                        // stage 1: the stage input is U^n itself
+                                        us[k] = a.rk_stage < 2 || !mine ? Real(0.0) : a.U[k * nc + idx];
+                                    }
+                                });
+
+        // ---- 5. divergence, fused RK stage and CFL rate
+        if (mine) {
 #pragma unroll
             for (int k = 0; k < 5; ++k) {
-                const Real u0 = a.U0[k * nc + idx];
-                Real o;
-                if (a.rk_stage == 1) {
-                    o = u0 + dt * r[k];  // the stage input is U^n itself: no second load
-                } else {
-                    const Real us = a.U[k * nc + idx];
-                    if (a.rk_stage == 2)
-                        o = Real(0.75) * u0 + Real(0.25) * (us + dt * r[k]);
-                    else
-                        o = u0 / Real(3.0) + Real(2.0) / Real(3.0) * (us + dt * r[k]);
-                }
-                un_[k] = o;
-                a.Uout[k * nc + idx] = o;
+                const Real fl = c == 0 ? L.sf[k][p] : sm[k][TL::mt(c - 1, p)];
+                r[k] = r[k] - (sm[k][TL::mt(c, p)] - fl) * a.inv_dx;
             }
-            if (a.want_rate) {
-                Real w[5];
-                to_prim(e, un_, w);
-                const Real c = sound_speed(e, w[0], w[4]);
-                Real ac = Real(-0.0);
+            if (a.rk_stage == 0) {
 #pragma unroll
-                for (int d = 0; d < 3; ++d)
-                    if (a.active[d]) ac += (fabs(w[1 + d]) + c) / a.dx_all[d];
-                rate = fmax(rate, (double)ac);
+                for (int k = 0; k < 5; ++k) a.R[k * nc + idx] = r[k];
+            } else {
+                Real uo[5];
+#pragma unroll
+                for (int k = 0; k < 5; ++k) {
+                    Real o;
+                    if (a.rk_stage == 1)
+                        o = u0[k] + dt * r[k];
+                    else if (a.rk_stage == 2)
+                        o = Real(0.75) * u0[k] + Real(0.25) * (us[k] + dt * r[k]);
+                    else
+                        o = u0[k] / Real(3.0) + Real(2.0) / Real(3.0) * (us[k] + dt * r[k]);
+                    uo[k] = o;
+                    a.Uout[k * nc + idx] = o;
+                }
+                if (a.want_rate) {
+                    Real w[5], v;
+                    to_prim_v(e, uo, w, v);
+                    const Real cs = sound_speed(e, w[0], w[4]);
+                    Real ac = Real(-0.0);
+#pragma unroll
+                    for (int d = 0; d < 3; ++d)
+                        if (a.active[d]) ac += (fabs(w[1 + d]) + cs) / a.dx_all[d];
+                    rate = fmax(rate, (double)ac);
+                }
             }
+        }
+        if constexpr (HYB) break;  // one tile (cut_segments)
+        // the cells the next tile takes over
+        if (c0 + T < s1) {
+            for (int it = tid; it < TL::HC * P; it += NT) {
+                const int h = CF ? it % TL::HC : it / P, hp = CF ? it / TL::HC : it % P;
+                const int q = TL::at(h, hp), o = TL::at(h + T, hp);
+#pragma unroll
+                for (int k = 0; k < 5; ++k) sw[k][q] = sw[k][o];
+                L.sre[q] = L.sre[o];
+            }
+            __syncthreads();
         }
     }
 
-    // ---- counters and rate: wave reduction, one atomic per workgroup
+    // ---- counters (per wave) and rate: one atomic per workgroup
+    if (a.want_rate) {
 #pragma unroll
-    for (int off = 32; off > 0; off >>= 1) {
-        n_shock += __shfl_xor(n_shock, off);
-        n_fb += __shfl_xor(n_fb, off);
-        n_lim += __shfl_xor(n_lim, off);
-        rate = fmax(rate, __shfl_xor(rate, off));
+        for (int off = 32; off > 0; off >>= 1) rate = fmax(rate, __shfl_xor(rate, off));
     }
     const int lane = tid & 63, wid = tid >> 6;
     if (lane == 0) {
         if (n_shock) atomicAdd(&scnt[0], n_shock);
-        if (n_fb) atomicAdd(&scnt[1], n_fb);
-        if (n_lim) atomicAdd(&scnt[2], n_lim);
         sred[wid] = rate;
     }
     __syncthreads();
@@ -251,98 +264,96 @@ __device__ __forceinline__ void axis_tile(const PassArgsT<Real>& a, int bid, Til
     }
 }
 
-template <int D, int MODE, int T, int P, int NT>
+template <int D, int MODE, int T, int P, bool CF, int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(EM_WAVES_PER_EU))) void axis_pass(PassArgs a) {
-    __shared__ TileLds<double, MODE, T, P, NT> L;
-    axis_tile<double, D, MODE, T, P, NT>(a, xcd_major((int)blockIdx.x, (int)gridDim.x), L);
+    __shared__ PassLds<double, MODE, T, P, CF, NT> L;
+    axis_segment<double, D, MODE, T, P, CF, NT>(a, xcd_major((int)blockIdx.x, (int)gridDim.x), L);
 }
 
 // The FP32 variant of the same pass (the reference's GpuSolver<f32>): state,
 // residual and arithmetic in float.
-template <int D, int MODE, int T, int P, int NT>
+template <int D, int MODE, int T, int P, bool CF, int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(EM_WAVES_PER_EU))) void axis_pass_f32(
     PassArgsT<float> a) {
-    __shared__ TileLds<float, MODE, T, P, NT> L;
-    axis_tile<float, D, MODE, T, P, NT>(a, xcd_major((int)blockIdx.x, (int)gridDim.x), L);
+    __shared__ PassLds<float, MODE, T, P, CF, NT> L;
+    axis_segment<float, D, MODE, T, P, CF, NT>(a, xcd_major((int)blockIdx.x, (int)gridDim.x), L);
 }
 
-// Ensemble pass: the tiles of every instance in one persistent launch.  Work
-// item w belongs to the instance i with prefix[i] <= w < prefix[i+1] and is
-// its tile w - prefix[i]; each instance brings its own arrays, extents,
+// Ensemble pass: the segments of every instance in one persistent launch.  Work
+// item w belongs to the instance i = owner[w] and is its segment
+// w - prefix[i]; each instance brings its own arrays, extents,
 // boundary conditions and device scalars (dt, CFL rate, counters).
-template <int D, int MODE, int T, int P, int NT>
+template <int D, int MODE, int T, int P, bool CF, int NT>
 __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(EM_WAVES_PER_EU))) void ens_pass(EnsPassArgs e) {
-    __shared__ TileLds<double, MODE, T, P, NT> L;
+    __shared__ PassLds<double, MODE, T, P, CF, NT> L;
     const XcdStride xs = xcd_stride();
     for (long long t = xs.first;; t += xs.step) {
         const long long w = xs.item(t);
         if (w >= e.total) break;
-        int lo = 0, hi = e.ninst;
-        while (hi - lo > 1) {
-            const int mid = (lo + hi) >> 1;
-            if (e.prefix[mid] <= w)
-                lo = mid;
-            else
-                hi = mid;
-        }
-        const PassArgs& a = e.args[lo];  // read in place (global memory, cached)
-        axis_tile<double, D, MODE, T, P, NT>(a, (int)(w - e.prefix[lo]), L);
+        const int i = __builtin_amdgcn_readfirstlane(scalar_copy(e.owner + w));
+        const PassArgs a = scalar_copy(e.args + i);
+        axis_segment<double, D, MODE, T, P, CF, NT>(a, (int)(w - scalar_copy(e.prefix + i)), L);
         __syncthreads();
     }
 }
 
+// One launch of tile shape (T, P): the layout of the LDS tile follows
+// whether the pass axis is contiguous (the last axis always is).
 template <int D, int MODE, int T, int P, int NT>
 static hipError_t launch_one(const PassArgs& a, hipStream_t s) {
-    const long long nblk = (long long)a.ntile * a.ngroup * a.n[a.slow_axis];
-    hipLaunchKernelGGL((axis_pass<D, MODE, T, P, NT>), dim3((unsigned)nblk), dim3(NT), 0, s, a);
+    const dim3 grid((unsigned)((long long)a.nseg * a.ngroup * a.n[a.slow_axis]));
+    if (D == 2 || a.dfast)
+        hipLaunchKernelGGL((axis_pass<D, MODE, T, P, true, NT>), grid, dim3(NT), 0, s, a);
+    else
+        hipLaunchKernelGGL((axis_pass<D, MODE, T, P, D == 2, NT>), grid, dim3(NT), 0, s, a);
     return hipGetLastError();
 }
 template <int D, int MODE, int T, int P, int NT>
 static hipError_t launch_one(const PassArgsT<float>& a, hipStream_t s) {
-    const long long nblk = (long long)a.ntile * a.ngroup * a.n[a.slow_axis];
-    hipLaunchKernelGGL((axis_pass_f32<D, MODE, T, P, NT>), dim3((unsigned)nblk), dim3(NT), 0, s, a);
+    const dim3 grid((unsigned)((long long)a.nseg * a.ngroup * a.n[a.slow_axis]));
+    if (D == 2 || a.dfast)
+        hipLaunchKernelGGL((axis_pass_f32<D, MODE, T, P, true, NT>), grid, dim3(NT), 0, s, a);
+    else
+        hipLaunchKernelGGL((axis_pass_f32<D, MODE, T, P, D == 2, NT>), grid, dim3(NT), 0, s, a);
     return hipGetLastError();
 }
 
 template <int D, int MODE, int T, int P, int NT>
 static hipError_t launch_ens_one(const EnsPassArgs& e, unsigned grid, hipStream_t s) {
-    hipLaunchKernelGGL((ens_pass<D, MODE, T, P, NT>), dim3(grid), dim3(NT), 0, s, e);
+    if (D == 2 || e.dfast)
+        hipLaunchKernelGGL((ens_pass<D, MODE, T, P, true, NT>), dim3(grid), dim3(NT), 0, s, e);
+    else
+        hipLaunchKernelGGL((ens_pass<D, MODE, T, P, D == 2, NT>), dim3(grid), dim3(NT), 0, s, e);
     return hipGetLastError();
 }
 
 // Tile table: must list the shapes of kTileCfgs (em_pass.h) in order.
+#define EM_FOR_TILE(CALL)                  \
+    switch (cfg) {                         \
+        case 0: return CALL(32, 8, 256);  \
+        case 1: return CALL(16, 16, 256);  \
+        case 2: return CALL(64, 8, 512);  \
+        case 3: return CALL(27, 8, 256);  \
+        case 4: return CALL(59, 4, 256);  \
+        case 5: return CALL(27, 4, 128);  \
+        case 6: return CALL(27, 2, 64);  \
+        case 7: return CALL(59, 1, 64);  \
+        case 8: return CALL(16, 4, 64);  \
+        case 9: return CALL(123, 4, 512);  \
+        default: return hipErrorInvalidValue; \
+    }
 template <int D, int MODE, class Args>
 static hipError_t launch_cfg(int cfg, const Args& a, hipStream_t s) {
-    switch (cfg) {
-        case 0: return launch_one<D, MODE, 32, 16, 640>(a, s);
-        case 1: return launch_one<D, MODE, 64, 8, 576>(a, s);
-        case 2: return launch_one<D, MODE, 128, 4, 576>(a, s);
-        case 3: return launch_one<D, MODE, 256, 2, 576>(a, s);
-        case 4: return launch_one<D, MODE, 27, 8, 256>(a, s);
-        case 5: return launch_one<D, MODE, 59, 4, 256>(a, s);
-        case 6: return launch_one<D, MODE, 59, 8, 512>(a, s);
-        case 7: return launch_one<D, MODE, 27, 16, 512>(a, s);
-        case 8: return launch_one<D, MODE, 123, 4, 512>(a, s);
-        case 9: return launch_one<D, MODE, 59, 16, 1024>(a, s);
-        default: return hipErrorInvalidValue;
-    }
+#define EM_CALL(T, P, NT) launch_one<D, MODE, T, P, NT>(a, s)
+    EM_FOR_TILE(EM_CALL)
+#undef EM_CALL
 }
 
 template <int D, int MODE>
 static hipError_t launch_ens_cfg(int cfg, const EnsPassArgs& e, unsigned grid, hipStream_t s) {
-    switch (cfg) {
-        case 0: return launch_ens_one<D, MODE, 32, 16, 640>(e, grid, s);
-        case 1: return launch_ens_one<D, MODE, 64, 8, 576>(e, grid, s);
-        case 2: return launch_ens_one<D, MODE, 128, 4, 576>(e, grid, s);
-        case 3: return launch_ens_one<D, MODE, 256, 2, 576>(e, grid, s);
-        case 4: return launch_ens_one<D, MODE, 27, 8, 256>(e, grid, s);
-        case 5: return launch_ens_one<D, MODE, 59, 4, 256>(e, grid, s);
-        case 6: return launch_ens_one<D, MODE, 59, 8, 512>(e, grid, s);
-        case 7: return launch_ens_one<D, MODE, 27, 16, 512>(e, grid, s);
-        case 8: return launch_ens_one<D, MODE, 123, 4, 512>(e, grid, s);
-        case 9: return launch_ens_one<D, MODE, 59, 16, 1024>(e, grid, s);
-        default: return hipErrorInvalidValue;
-    }
+#define EM_CALL(T, P, NT) launch_ens_one<D, MODE, T, P, NT>(e, grid, s)
+    EM_FOR_TILE(EM_CALL)
+#undef EM_CALL
 }
 
 // This translation unit instantiates one flux mode (EM_MODE).

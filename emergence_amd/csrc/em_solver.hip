@@ -207,7 +207,7 @@ struct Grid {
     double bc_state[3][2][5];
     int mode, positivity;
     double cfl, tol;
-    int cfg[3] = {6, 6, 6};
+    int cfg[3] = {0, 0, 0};
     long long ncell;
     long long stride[3];
     int nactive;
@@ -254,6 +254,7 @@ struct Grid {
         stride[0] = n[1] * n[2];
         stride[1] = n[2];
         stride[2] = 1;
+        for (int d = 0; d < 3; ++d) cfg[d] = default_cfg(d);
     }
 
     PassArgs pass_args(int d, DevScalars* sc) const { return pass_args_t<double>(d, sc); }
@@ -291,11 +292,45 @@ struct Grid {
             a.fast_axis = t[0];
             a.slow_axis = t[1];
         }
+        a.n_fast = a.n[a.fast_axis];
+        a.s_fast = a.stride[a.fast_axis];
+        a.s_slow = a.stride[a.slow_axis];
         a.dfast = stride[d] == 1 ? 1 : 0;
         const TileCfg tc = kTileCfgs[cfg[d]];
-        a.ntile = (int)((n[d] + tc.T - 1) / tc.T);
         a.ngroup = (int)((n[a.fast_axis] + tc.P - 1) / tc.P);
+        cut_segments(a, d, mode, cfg[d]);
         return a;
+    }
+
+    // Segments of a pass along d with tile shape cfg.  Long segments share most (see em_faces.h); the launch
+    // still has to fill the GPU (256 CUs of 16 waves) twice over so that its
+    // last round weighs little.  Hybrid: single tiles.
+    template <class Real>
+    static void cut_segments(PassArgsT<Real>& a, int d, int mode, int cfg) {
+        const long long groups = (long long)a.ngroup * a.n[a.slow_axis];
+        const TileCfg tc = kTileCfgs[cfg];
+        const long long resident = 256ll * 16 * 64 / tc.NT;
+        const int ntile = (a.n[d] + tc.T - 1) / tc.T;
+        const long long want = (2 * resident + groups - 1) / groups;
+        const int per = mode == MODE_HYBRID ? 1 : (int)std::max<long long>(1, ntile / std::min<long long>(want, ntile));
+        a.seg = per * tc.T;
+        a.nseg = (a.n[d] + a.seg - 1) / a.seg;
+    }
+
+    // Tile shape of axis d before any autotuning, by the number of 27 x 8
+    // tiles of the grid (256^3 has 81,920 an axis, 512^2 1,216, 64^2 24).
+    // Where they fill the GPU four times over, Weno segments of many 32-cell
+    // tiles, one thread per cell (256^3: 1.04 ms an axis against 1.19 ms in
+    // 27-cell tiles); below, and in Hybrid mode, single tiles, one thread per
+    // midpoint (512^2: 29-33 us against 31-34); and a few one-wave tiles for
+    // the smallest grids, whose time is one tile's latency (64^2 Hybrid: 16
+    // us against 16-21).
+    int default_cfg(int d) const {
+        const int f = active(d == 2 ? 1 : 2) ? (d == 2 ? 1 : 2) : (d == 0 ? 1 : 0);
+        const long long tiles = (n[d] + 26) / 27 * ((n[f] + 7) / 8) * (ncell / n[d] / n[f]);
+        if (tiles < 256) return 6;
+        if (mode == MODE_HYBRID) return 3;
+        return tiles < 4096 ? (stride[d] == 1 ? 4 : 3) : 0;
     }
 
     uint64_t faces_per_stage() const {
@@ -345,9 +380,6 @@ struct SolverCore : Grid {
         h[0].active = 1;
         HIPCHK(hipMemcpyAsync(sc, h.data(), sizeof(DevScalars), hipMemcpyHostToDevice, stream));
         HIPCHK(hipStreamSynchronize(stream));
-        // default tile: 59 cells x 8 pencils, 512 threads (one midpoint per
-        // thread, two workgroups per CU); the autotuner may pick another
-        for (int d = 0; d < 3; ++d) cfg[d] = 6;
     }
 
     ~SolverCore() {
@@ -1151,14 +1183,16 @@ __global__ void k_ens_copy(const CopyTask* __restrict__ t) {
 struct Ensemble {
     std::vector<Solver*> in;
     int n = 0;
-    int mode, cfg = 6, precise = 1;
+    int mode, cfg = 4, precise = 1;
     bool batched = true;
     double cfl;
     hipStream_t stream = nullptr;
     DevScalars** d_scs = nullptr;
     PassArgs* d_args[3][3] = {};
     long long* d_prefix[3][3] = {};
+    int* d_owner[3] = {};  // instance of each work item of an axis (the same in every stage)
     long long total[3][3] = {};
+    int dfast[3] = {};
     long long* d_step = nullptr;
     hipGraphExec_t graph = nullptr;
     int graph_key = -1;
@@ -1225,6 +1259,10 @@ struct Ensemble {
                 d_args[sidx][d] = nullptr;
                 d_prefix[sidx][d] = nullptr;
             }
+        for (auto& p : d_owner) {
+            f(p);
+            p = nullptr;
+        }
         f(d_scs);
         f(d_step);
         f(d_copy);
@@ -1265,6 +1303,8 @@ struct Ensemble {
             for (int d = 0; d < 3; ++d) {
                 std::vector<PassArgs> a;
                 std::vector<long long> pre(1, 0);
+                for (int i = 0; i < n; ++i)
+                    if (in[i]->active(d)) dfast[d] = in[i]->pass_args(d).dfast;
                 for (int i = 0; i < n; ++i) {
                     Solver& S = *in[i];
                     if (!S.active(d)) {
@@ -1291,7 +1331,7 @@ struct Ensemble {
                     p.stage_dt_host = 0;
                     p.stage_dt = 0.0;
                     a.push_back(p);
-                    pre.push_back(pre.back() + (long long)p.ntile * p.ngroup * p.n[p.slow_axis]);
+                    pre.push_back(pre.back() + (long long)p.nseg * p.ngroup * p.n[p.slow_axis]);
                 }
                 total[st - 1][d] = pre.back();
                 if (d_args[st - 1][d]) HIPCHK(hipFree(d_args[st - 1][d]));
@@ -1301,6 +1341,15 @@ struct Ensemble {
                 HIPCHK(hipMemcpyAsync(d_args[st - 1][d], a.data(), sizeof(PassArgs) * n, hipMemcpyHostToDevice, stream));
                 HIPCHK(hipMemcpyAsync(d_prefix[st - 1][d], pre.data(), sizeof(long long) * (n + 1),
                                       hipMemcpyHostToDevice, stream));
+                std::vector<int> own;
+                if (st == 1 && pre.back() > 0) {
+                    own.resize(pre.back());
+                    for (int i = 0; i < n; ++i) std::fill(own.begin() + pre[i], own.begin() + pre[i + 1], i);
+                    if (d_owner[d]) HIPCHK(hipFree(d_owner[d]));
+                    d_owner[d] = nullptr;
+                    HIPCHK(hipMalloc(&d_owner[d], sizeof(int) * own.size()));
+                    HIPCHK(hipMemcpyAsync(d_owner[d], own.data(), sizeof(int) * own.size(), hipMemcpyHostToDevice, stream));
+                }
                 HIPCHK(hipStreamSynchronize(stream));
             }
         graph_key = -1;
@@ -1361,7 +1410,7 @@ struct Ensemble {
         for (int d = 0; d < 3; ++d) {
             if (total[st - 1][d] == 0) continue;
             if (batched) {
-                EnsPassArgs e{d_args[st - 1][d], d_prefix[st - 1][d], n, total[st - 1][d]};
+                EnsPassArgs e{d_args[st - 1][d], d_prefix[st - 1][d], d_owner[d], dfast[d], total[st - 1][d]};
                 const unsigned grid = (unsigned)std::min<long long>(total[st - 1][d], 4096);
                 HIPCHK(precise ? precise::launch_ens_pass(d, mode, cfg, e, grid, stream)
                                : fast::launch_ens_pass(d, mode, cfg, e, grid, stream));
@@ -1805,7 +1854,7 @@ static void rhs_noalloc(const Grid& G, int precise, double stage_dt, const doubl
     for (int d = 0; d < 3; ++d) {
         if (!G.active(d)) continue;
         const PassArgs a = G.pass_args(d, nullptr);
-        const long long nblk = (long long)a.ntile * a.ngroup * a.n[a.slow_axis];
+        const long long nblk = (long long)a.nseg * a.ngroup * a.n[a.slow_axis];
         if (nblk > 0x7fffffffll) throw Error(EM_ERR_ARG, "mesh too large for one axis-pass launch");
     }
     DevScalars* sc = noalloc_scratch();

@@ -55,19 +55,22 @@ struct PassArgsT {
     int rk_stage;          // 0: store residual only; 1..3: fused SSP-RK3 stage
     int want_rate;         // accumulate the CFL rate of the RK output
     int fast_axis, slow_axis;
+    int n_fast;            // n and strides of those axes (no indexed reads in the kernels)
+    long long s_fast, s_slow;
     int dfast;             // stride along the pass axis is 1
-    int ntile, ngroup;     // tiles along the axis, pencil groups along fast_axis
+    int seg, nseg, ngroup; // cells of a segment, segments along the axis, pencil groups along fast_axis
     int stage_dt_host;     // 0: lambda from sc->dt
     double stage_dt;       // used when stage_dt_host != 0
 };
 using PassArgs = PassArgsT<double>;
 
-// Ensemble pass: per-instance pass arguments and the prefix sums of the
-// instances' tile counts (ninst + 1 entries; total = prefix[ninst]).
+// Ensemble pass: per-instance pass arguments, the prefix sums of the
+// instances' segment counts and each segment's instance (ninst + 1 entries; total = prefix[ninst]).
 struct EnsPassArgs {
     const PassArgs* args;
     const long long* prefix;
-    int ninst;
+    const int* owner;  // instance of every work item
+    int dfast;  // the pass axis is contiguous (of every instance with work)
     long long total;
 };
 

@@ -27,6 +27,7 @@
 
 #include "../../include/em_hip.h"
 #include "em_fiveeq.h"
+#include "em_hostio.h"
 #include "em_types.h"
 
 namespace em {
@@ -671,6 +672,8 @@ struct FeCore {
         FECHK(hipMemcpyAsync(sc, h.data(), sizeof(FeScalars), hipMemcpyHostToDevice, stream));
         FECHK(hipStreamSynchronize(stream));
     }
+    HostIo<7> io;  // conversion buffer of upload, download and rhs
+
     ~FeCore() {
         for (auto* b : U)
             if (b) (void)hipFree(b);
@@ -679,35 +682,12 @@ struct FeCore {
         if (stream) (void)hipStreamDestroy(stream);
     }
 
-    void upload(const double* u) {
-        std::vector<Real> h(7 * ncell);
-        const int m1 = m(1), m2 = m(2);
-        for (long long i = 0; i < n[0]; ++i)
-            for (long long j = 0; j < n[1]; ++j)
-                for (long long k = 0; k < n[2]; ++k) {
-                    const long long q = ((i + g(0)) * m1 + (j + g(1))) * m2 + (k + g(2));
-                    const long long c = (i * n[1] + j) * n[2] + k;
-                    for (int v = 0; v < 7; ++v) h[v * ncell + c] = Real(u[q * 7 + v]);
-                }
-        FECHK(hipMemcpyAsync(U[0], h.data(), sizeof(Real) * 7 * ncell, hipMemcpyHostToDevice, stream));
-        FECHK(hipStreamSynchronize(stream));
+    HostLayout host_layout() const {
+        return HostLayout{n[0], n[1], n[2], m(1), m(2), g(0), g(1), g(2), ncell, (long long)m(0) * m(1) * m(2)};
     }
+    void upload(const double* u) { FECHK(io.in(host_layout(), u, U[0], stream)); }
     // ghost-padded AoS with the interior filled and zero ghosts
-    void to_host(const Real* dev, double* u) {
-        std::vector<Real> h(7 * ncell);
-        FECHK(hipMemcpyAsync(h.data(), dev, sizeof(Real) * 7 * ncell, hipMemcpyDeviceToHost, stream));
-        FECHK(hipStreamSynchronize(stream));
-        const long long L = (long long)m(0) * m(1) * m(2);
-        std::fill(u, u + 7 * L, 0.0);
-        const int m1 = m(1), m2 = m(2);
-        for (long long i = 0; i < n[0]; ++i)
-            for (long long j = 0; j < n[1]; ++j)
-                for (long long k = 0; k < n[2]; ++k) {
-                    const long long q = ((i + g(0)) * m1 + (j + g(1))) * m2 + (k + g(2));
-                    const long long c = (i * n[1] + j) * n[2] + k;
-                    for (int v = 0; v < 7; ++v) u[q * 7 + v] = (double)h[v * ncell + c];
-                }
-    }
+    void to_host(const Real* dev, double* u) { FECHK(io.out(host_layout(), dev, false, u, stream)); }
 
     FePassArgsT<Real> pass_args(int d) const {
         FePassArgsT<Real> a{};

@@ -20,6 +20,7 @@
 
 #include "../../include/em_hip.h"
 #include "em_adjoint.h"
+#include "em_hostio.h"
 #include "em_pass.h"
 #include "em_types.h"
 
@@ -353,6 +354,7 @@ struct SolverCore : Grid {
     Real* U[3] = {nullptr, nullptr, nullptr};  // U^n, stage 1, stage 2
     Real* R = nullptr;
     Real* pad = nullptr;
+    HostIo<5> io;  // conversion buffer of upload, download and the host-array entry points
     Real* bcdev = nullptr;  // [3][2][5] boundary states for the ghost sweep
     double* dt_hist = nullptr;  // device dt history of a CFL-driven forward run
     int64_t dt_hist_cap = 0;
@@ -396,18 +398,10 @@ struct SolverCore : Grid {
         if (rstream) (void)hipStreamDestroy(rstream);
     }
 
+    HostLayout host_layout() const { return HostLayout{n[0], n[1], n[2], m(1), m(2), g(0), g(1), g(2), ncell, len()}; }
+
     void upload(const double* u) {
-        std::vector<Real> h(5 * ncell);
-        const int m1 = m(1), m2 = m(2);
-        for (long long i = 0; i < n[0]; ++i)
-            for (long long j = 0; j < n[1]; ++j)
-                for (long long k = 0; k < n[2]; ++k) {
-                    const long long q = ((i + g(0)) * m1 + (j + g(1))) * m2 + (k + g(2));
-                    const long long c = (i * n[1] + j) * n[2] + k;
-                    for (int v = 0; v < 5; ++v) h[v * ncell + c] = Real(u[q * 5 + v]);
-                }
-        HIPCHK(hipMemcpyAsync(U[0], h.data(), sizeof(Real) * 5 * ncell, hipMemcpyHostToDevice, stream));
-        HIPCHK(hipStreamSynchronize(stream));
+        HIPCHK(io.in(host_layout(), u, U[0], stream));
         rate_valid = false;
     }
 
@@ -448,12 +442,7 @@ struct SolverCore : Grid {
 
     void download(double* u) {
         fill_pad();
-        const long long L = len();
-        std::vector<Real> h(5 * L);
-        HIPCHK(hipMemcpyAsync(h.data(), pad, sizeof(Real) * 5 * L, hipMemcpyDeviceToHost, stream));
-        HIPCHK(hipStreamSynchronize(stream));
-        for (long long q = 0; q < L; ++q)
-            for (int v = 0; v < 5; ++v) u[q * 5 + v] = (double)h[v * L + q];
+        HIPCHK(io.out(host_layout(), pad, true, u, stream));
     }
 
     PassArgsT<Real> pass_args(int d) const { return Grid::pass_args_t<Real>(d, sc); }
@@ -557,19 +546,8 @@ struct SolverCore : Grid {
         Scalars before = read_scalars();
         reset_run(0.0);
         stage(U[0], nullptr, 0, false, 1, stage_dt, nullptr);
-        std::vector<Real> h(5 * ncell);
-        HIPCHK(hipMemcpyAsync(h.data(), R, sizeof(Real) * 5 * ncell, hipMemcpyDeviceToHost, stream));
         Scalars after = read_scalars();
-        const long long L = len();
-        std::fill(out, out + 5 * L, 0.0);
-        const int m1 = m(1), m2 = m(2);
-        for (long long i = 0; i < n[0]; ++i)
-            for (long long j = 0; j < n[1]; ++j)
-                for (long long k = 0; k < n[2]; ++k) {
-                    const long long q = ((i + g(0)) * m1 + (j + g(1))) * m2 + (k + g(2));
-                    const long long c = (i * n[1] + j) * n[2] + k;
-                    for (int v = 0; v < 5; ++v) out[q * 5 + v] = (double)h[v * ncell + c];
-                }
+        HIPCHK(io.out(host_layout(), R, false, out, stream));
         if (stats) {
             stats[0] = faces_per_stage();
             for (int q = 0; q < 3; ++q) stats[1 + q] = after.counters[q] - before.counters[q];
@@ -839,34 +817,8 @@ struct Solver : SolverCore<double> {
         }
     }
 
-    void host_to_soa(const double* u, double* dev) {
-        std::vector<double> h(5 * ncell);
-        const int m1 = m(1), m2 = m(2);
-        for (long long i = 0; i < n[0]; ++i)
-            for (long long j = 0; j < n[1]; ++j)
-                for (long long k = 0; k < n[2]; ++k) {
-                    const long long q = ((i + g(0)) * m1 + (j + g(1))) * m2 + (k + g(2));
-                    const long long c = (i * n[1] + j) * n[2] + k;
-                    for (int v = 0; v < 5; ++v) h[v * ncell + c] = u[q * 5 + v];
-                }
-        HIPCHK(hipMemcpyAsync(dev, h.data(), sizeof(double) * 5 * ncell, hipMemcpyHostToDevice, stream));
-        HIPCHK(hipStreamSynchronize(stream));
-    }
-
-    void soa_to_host(const double* dev, double* u) {
-        std::vector<double> h(5 * ncell);
-        HIPCHK(hipMemcpyAsync(h.data(), dev, sizeof(double) * 5 * ncell, hipMemcpyDeviceToHost, stream));
-        HIPCHK(hipStreamSynchronize(stream));
-        std::fill(u, u + 5 * len(), 0.0);
-        const int m1 = m(1), m2 = m(2);
-        for (long long i = 0; i < n[0]; ++i)
-            for (long long j = 0; j < n[1]; ++j)
-                for (long long k = 0; k < n[2]; ++k) {
-                    const long long q = ((i + g(0)) * m1 + (j + g(1))) * m2 + (k + g(2));
-                    const long long c = (i * n[1] + j) * n[2] + k;
-                    for (int v = 0; v < 5; ++v) u[q * 5 + v] = h[v * ncell + c];
-                }
-    }
+    void host_to_soa(const double* u, double* dev) { HIPCHK(io.in(host_layout(), u, dev, stream)); }
+    void soa_to_host(const double* dev, double* u) { HIPCHK(io.out(host_layout(), dev, false, u, stream)); }
 
     void ensure_adjbuf() {
         if (!adjbuf) HIPCHK(hipMalloc(&adjbuf, sizeof(double) * 20 * ncell));

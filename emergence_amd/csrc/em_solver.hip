@@ -87,29 +87,39 @@ __global__ void k_record_dt(const DevScalars* sc, double* hist) {
 //   run_to == 1: Solver::run_to rule (solver.rs:758-768): stop once
 //                t >= t_end - 1e-10 |t_end|; dt = min(cfl / rate, t_end - t);
 //                collapse if dt is not finite or <= 1e-12 max(|t_end|, 1e-300)
-__global__ void k_dt_from_rate(DevScalars* sc, double cfl, int run_to) {
+// One wave, a lane per rate slot (a single thread reading the 64 slots in
+// turn took 5 to 6 us, a third of a small grid's axis pass); clears the slots
+// for the step's last stage.
+__global__ __launch_bounds__(kSlots) void k_dt_from_rate(DevScalars* sc, double cfl, int run_to) {
+    static_assert(kSlots == 64, "one wave");
     if (sc->active == 0) return;
-    const double rate = __longlong_as_double((long long)rate_bits(sc));
+    const int lane = threadIdx.x;
+    double rate = __longlong_as_double((long long)sc->rate[lane][0]);
+#pragma unroll
+    for (int off = 32; off > 0; off >>= 1) rate = fmax(rate, __shfl_xor(rate, off));
     double dt = cfl / rate;
+    bool go = true;
+    int err = 0;
     if (run_to) {
         const double te = sc->t_end;
         if (!(sc->t < te - 1e-10 * fabs(te))) {
-            sc->active = 0;
-            return;
-        }
-        dt = fmin(dt, te - sc->t);
-        if (!(isfinite(dt) && dt > 1e-12 * fmax(fabs(te), 1e-300))) {
-            sc->err |= 1;
-            sc->active = 0;
-            return;
+            go = false;
+        } else {
+            dt = fmin(dt, te - sc->t);
+            if (!(isfinite(dt) && dt > 1e-12 * fmax(fabs(te), 1e-300))) err = 1;
         }
     } else if (!(isfinite(dt) && dt > 0.0)) {
-        sc->err |= 1;
-        sc->active = 0;
+        err = 1;
+    }
+    if (!go || err) {
+        if (lane == 0) {
+            if (err) sc->err |= 1;
+            sc->active = 0;
+        }
         return;
     }
-    sc->dt = dt;
-    for (int i = 0; i < kSlots; ++i) sc->rate[i][0] = 0ull;
+    if (lane == 0) sc->dt = dt;
+    sc->rate[lane][0] = 0ull;
 }
 
 // CFL rate max over interior cells: dt_cfl (solver.rs:478-523).  Wave
@@ -484,13 +494,14 @@ struct SolverCore : Grid {
     // U1 = U + dt L(U); U2 = 3/4 U + 1/4 (U1 + dt L(U1));
     // U <- U/3 + 2/3 (U2 + dt L(U2)), the last stage also leaving the CFL
     // rate of the new state in sc->rate.
-    void step_kernels(std::vector<hipEvent_t>* evs = nullptr) {
+    // zero_rate = false: k_dt_from_rate has cleared the slots.
+    void step_kernels(std::vector<hipEvent_t>* evs = nullptr, bool zero_rate = true) {
         hipEvent_t* e[3] = {nullptr, nullptr, nullptr};
         if (evs)
             for (int s = 0; s < 3; ++s) e[s] = evs->data() + 6 * s;
         stage(U[0], U[1], 1, false, 0, 0.0, e[0]);
         stage(U[1], U[2], 2, false, 0, 0.0, e[1]);
-        hipLaunchKernelGGL(k_zero_rate, dim3(1), dim3(kSlots), 0, stream, sc);
+        if (zero_rate) hipLaunchKernelGGL(k_zero_rate, dim3(1), dim3(kSlots), 0, stream, sc);
         stage(U[2], U[0], 3, true, 0, 0.0, e[2]);
         hipLaunchKernelGGL(k_advance, dim3(1), dim3(1), 0, stream, sc);
         HIPCHK(hipGetLastError());
@@ -586,9 +597,9 @@ struct SolverCore : Grid {
     // One step driven by device-resident dt: dt kernel + stages + advance.
     // Mode 2 (forward run) also records dt in dt_hist[steps].
     void device_step(int run_mode) {
-        hipLaunchKernelGGL(k_dt_from_rate, dim3(1), dim3(1), 0, stream, sc, cfl, run_mode == 1 ? 1 : 0);
+        hipLaunchKernelGGL(k_dt_from_rate, dim3(1), dim3(kSlots), 0, stream, sc, cfl, run_mode == 1 ? 1 : 0);
         if (run_mode == 2) hipLaunchKernelGGL(k_record_dt, dim3(1), dim3(1), 0, stream, sc, dt_hist);
-        step_kernels();
+        step_kernels(nullptr, false);
     }
 
     hipGraphExec_t get_graph(int run_mode) {
@@ -634,7 +645,7 @@ struct SolverCore : Grid {
             for (auto& x : ev) HIPCHK(hipEventCreate(&x));
             for (int64_t q = 0; q < nsteps; ++q) {
                 std::vector<hipEvent_t> step_ev(ev.begin() + 18 * q, ev.begin() + 18 * (q + 1));
-                hipLaunchKernelGGL(k_dt_from_rate, dim3(1), dim3(1), 0, stream, sc, cfl, 0);
+                hipLaunchKernelGGL(k_dt_from_rate, dim3(1), dim3(kSlots), 0, stream, sc, cfl, 0);
                 step_kernels(&step_ev);
             }
             HIPCHK(hipStreamSynchronize(stream));
@@ -933,7 +944,7 @@ struct Solver : SolverCore<double> {
             if (all) {
                 // device_step(2) on the kept buffers
                 for (int64_t s = 0; s < nsteps; ++s) {
-                    hipLaunchKernelGGL(k_dt_from_rate, dim3(1), dim3(1), 0, stream, sc, cfl, 0);
+                    hipLaunchKernelGGL(k_dt_from_rate, dim3(1), dim3(kSlots), 0, stream, sc, cfl, 0);
                     hipLaunchKernelGGL(k_record_dt, dim3(1), dim3(1), 0, stream, sc, dt_hist);
                     kept_step(s);
                 }

@@ -1,11 +1,12 @@
 // Fused per-axis pass of the compressible RHS on gfx950.
 //
-// One workgroup owns a tile of T cells along the pass axis D times P
-// neighbouring pencils.  Phases (LDS-staged, one barrier between each):
-//   1. load: coalesced SoA loads of the 5 conserved variables of the T+10
-//      cells (5-cell halo on each side; ghost cells are produced from the
-//      boundary condition of the pencil itself), conversion to primitives
-//      into LDS (plus the hybrid sensor ln rho, ln(p + p_inf));
+// One workgroup owns a segment of P neighbouring pencils along the pass axis
+// D and walks it in tiles of T cells (em_faces.h).  Phases of a tile
+// (LDS-staged, one barrier between each):
+//   1. load: coalesced SoA loads of the 5 conserved variables of the tile's
+//      cells and, in the first tile, its halo of 10 (ghost cells are produced
+//      from the boundary condition of the pencil itself), conversion to
+//      primitives into LDS (plus the hybrid sensor ln rho, ln(p + p_inf));
 //   2. hybrid only: blend weight theta of every face;
 //   3. WCNS midpoints: each of the T+5 midpoints of a pencil is computed
 //      once (characteristic WENO5-Z interpolation + HLLC) into LDS;
@@ -23,6 +24,12 @@
 // with -ffp-contract=off (reproduces the reference CPU arithmetic) or
 // EM_VARIANT=fast with FMA contraction; EM_MODE = 0 hybrid, 1 weno,
 // 2 central.  Kernels ask for 4 waves per SIMD (<= 128 VGPRs).
+//
+// Bound by FP64 instruction issue (VALU 81 to 85% busy).  256^3 Weno, x, y and
+// z pass of a step: 1.58, 1.60, 1.76 ms with independent 59-cell tiles and
+// general divisions (2,544 VALU instructions per cell along x), 1.03, 1.04,
+// 1.13 ms now (about 1,800).  Code size counts: a version that inlined the
+// boundary images three times (59 KB) ran 20% slower than this one.
 #include <hip/hip_runtime.h>
 
 #include "em_pass.h"

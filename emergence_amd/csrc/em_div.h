@@ -95,7 +95,8 @@ __device__ __forceinline__ double rcp3_mid(double d0, double d1, double d2, doub
     r2 = rcp_step(d2, r * p);
     return pp;
 }
-// the same for two doubles of [2^-1, 2^480]
+// the same for two doubles of at least 2^-1 (NaN where their product overflows;
+// div_by_fix then makes the quotients infinite)
 __device__ __forceinline__ void rcp2_mid(double d0, double d1, double& r0, double& r1) {
     const double p = d0 * d1;
     const double r = rcp_step(p, __builtin_amdgcn_rcp(p));

@@ -47,6 +47,14 @@ def _state(n, kind, seed=5, ng=6):
     elif kind == "cold":  # kinetic energy far above the internal one: the limiter's test is near its margin
         p = p * 1e-9
         vel = vel + 5.0
+    elif kind == "outlier":  # gas at rest but for single cells far out: the product of two weight sums overflows
+        # (seven cells apart along every axis, one component each, density 1: the pressure there is exactly zero)
+        vel *= 0.0
+        i, j, k = np.indices(n)
+        comp = np.where((i + 3 * j + 5 * k) % 7 == 0, (i + j + k) % 3, -1)
+        rho = np.where(comp >= 0, 1.0, rho)
+        for d in range(3):
+            vel[d][comp == d] = 2.0 ** 70
     u = np.zeros(tuple(v + 2 * ng if v > 1 else 1 for v in n) + (5,))
     g = [ng if v > 1 else 0 for v in n]
     ui = u[g[0]:g[0] + n[0], g[1]:g[1] + n[1], g[2]:g[2] + n[2]]
@@ -59,7 +67,7 @@ def _state(n, kind, seed=5, ng=6):
 
 @pytest.mark.parametrize("mode", ["weno", "central"])
 @pytest.mark.parametrize("n", [(67, 9, 1), (12, 10, 70), (1, 70, 5)])
-@pytest.mark.parametrize("kind", ["fronts", "signed_zero", "small", "large", "near_vacuum", "cold"])
+@pytest.mark.parametrize("kind", ["fronts", "signed_zero", "small", "large", "near_vacuum", "cold", "outlier"])
 def test_residual_bits_in_and_outside_the_mid_range(em, kind, n, mode):
     bc = [["outflow", "outflow"], ["periodic", "periodic"], ["reflect", "outflow"]]
     u = _state(n, kind)

@@ -126,14 +126,14 @@ __device__ __forceinline__ void to_prim_v(const EosT<R>& e, const R u[5], R w[5]
     } else {
         const R r = rcp_mid(rho);
         v = inv_by(rho, r);
-        const R vx = div_by(u[1], rho, r), vy = div_by(u[2], rho, r), vz = div_by(u[3], rho, r);
-        const R en = div_by(u[4], rho, r) - R(0.5) * (vx * vx + vy * vy + vz * vz);
+        const R vx = div_by_pos(u[1], rho, r), vy = div_by_pos(u[2], rho, r), vz = div_by_pos(u[3], rho, r);
+        const R en = div_by_pos(u[4], rho, r) - R(0.5) * (vx * vx + vy * vy + vz * vz);
         w[0] = rho;
         w[1] = vx;
         w[2] = vy;
         w[3] = vz;
         const R a = (e.gamma - R(1.0)) * (en - e.q), vb = v - e.b;
-        w[4] = div_by(a, vb, rcp_volume(e, rho, vb)) - e.gamma * e.p_inf;
+        w[4] = div_by_pos(a, vb, rcp_volume(e, rho, vb)) - e.gamma * e.p_inf;
         // an overflowing quotient leaves p infinite or NaN
         if (!in_mid(rho) || !in_mid(vb) || too_small(u[1]) || too_small(u[2]) || too_small(u[3]) || too_small(u[4]) ||
             too_small(a) || !(fabs(w[4]) <= Mid<R>::huge)) {
@@ -150,7 +150,7 @@ __device__ __forceinline__ R eos_rho_e_v(const EosT<R>& e, R rho, R p, R v) {
         return eos_rho_e(e, rho, p);
     } else {
         const R a = (p + e.gamma * e.p_inf) * (v - e.b);
-        R x = div_by(a, e.gamma - R(1.0), e.rg);
+        R x = div_by_pos(a, e.gamma - R(1.0), e.rg);
         if (too_small(a) || !(fabs(x) <= Mid<R>::huge)) x = a / (e.gamma - R(1.0));
         return rho * (x + e.q);
     }

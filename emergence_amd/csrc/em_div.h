@@ -10,8 +10,9 @@
 // quotient of one divisor (and, through products, by several divisors).
 // div_by is that core: with r = 1/b to within about half an ulp,
 //   q = RN(a r),  rem = a - b q (exact),  RN(q + rem r) = RN(a / b).
-// It needs |b|, |a| and |a/b| within 2^+-900 (or a = +0).  The callers test
-// their operands (Mid) and hand everything else to the general expressions.
+// It needs |b|, |a| and |a/b| within 2^+-900 (or a = +0; div_by_pos and
+// div_by_fix also keep the sign of -0).  The callers test their operands (Mid)
+// and hand everything else to the general expressions.
 #pragma once
 #include <hip/hip_runtime.h>
 
@@ -64,6 +65,9 @@ __device__ __forceinline__ double div_by(double a, double b, double r) {
 __device__ __forceinline__ double div_by_fix(double a, double b, double r) {
     return __builtin_amdgcn_div_fixup(div_by(a, b, r), b, a);
 }
+// a / b, b > 0: div_by with the sign of a zero dividend (div_by turns -0 into
+// +0; a reflecting wall makes -0 of every zero momentum)
+__device__ __forceinline__ double div_by_pos(double a, double b, double r) { return copysign(div_by(a, b, r), a); }
 // 1 / b from r = rcp_mid(b)
 __device__ __forceinline__ double inv_by(double b, double r) { return rcp_step(b, r); }
 

@@ -40,6 +40,23 @@ static double value(bool wide) {
 static const Eos gases[] = {Eos{1.4, 0, 0, 0}, Eos{5.0 / 3.0, 0, 0, 0}, Eos{4.4, 0.6, 0, 0.1}, Eos{1.3, 0.2, 0.3, 0},
                             Eos{1.3, 0.2, 0.3, -0.1}};
 
+static void check_to_prim(int n) {
+    for (int i = 0; i < n; ++i) {
+        const Eos e = gases[pick(5)];
+        const bool wide = pick(4) == 0;
+        double u[5] = {std::fabs(value(wide)), value(wide), value(wide), value(wide), value(wide)};
+        if (pick(2)) u[0] = uni(0.1, 3.0), u[4] = uni(0.1, 9.0);
+        double w[5], g[5], v;
+        to_prim_v(e, u, w, v);
+        to_prim(e, u, g);
+        for (int k = 0; k < 5; ++k)
+            if (!same(w[k], g[k])) report("to_prim", u, 5, w[k], g[k]);
+        if (!same(v, 1.0 / u[0])) report("1 / rho", u, 1, v, 1.0 / u[0]);
+        const double x = eos_rho_e_v(e, g[0], g[4], v), y = eos_rho_e(e, g[0], g[4]);
+        if (!same(x, y)) report("rho_e", u, 5, x, y);
+    }
+}
+
 static void pair_case(const double v[6], long long& taken) {
     double l, r;
     unsigned top = 0;
@@ -174,6 +191,7 @@ static void check_admissible(int n) {
 }
 
 int main() {
+    check_to_prim(400000);
     check_pairs(400000);
     check_midpoints<0>(150000);
     check_midpoints<1>(150000);

@@ -20,7 +20,7 @@ namespace EM_VARIANT {
 
 // LDS of one work item (whole pencils of a B-cell block, P of them)
 template <class Real, int MODE, int B, int P>
-using AmrLds = Tile<Real, MODE, B, P, false>;
+using AmrLds = Tile<Real, MODE, B, P, false, false>;
 
 // Work item w of one batched AMR pass: the pencil group w % ngroup of leaf
 // leaf0 + w / ngroup (every thread of the workgroup calls it; it returns
@@ -95,8 +95,8 @@ __device__ __forceinline__ void amr_item(const AmrPassArgsT<Real>& pa, long long
         for (int q = 0; q < 5; ++q) L.sw[q][TL::at(c, p)] = wv[q];
         L.sre[TL::at(c, p)] = eos_rho_e_v(e, wv[0], wv[4], v);
         if constexpr (HYB) {
-            L.ss[0][TL::at(c, p)] = log(fmax(wv[0], Real(1e-300)));
-            L.ss[1][TL::at(c, p)] = log(fmax(wv[4] + e.p_inf, Real(1e-300)));
+            L.ss[0][TL::st(c, p)] = log(fmax(wv[0], Real(1e-300)));
+            L.ss[1][TL::st(c, p)] = log(fmax(wv[4] + e.p_inf, Real(1e-300)));
         }
     }
     __syncthreads();

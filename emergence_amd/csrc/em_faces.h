@@ -19,6 +19,12 @@
 // if one of its faces m - 4 .. m has theta > 0; the weights of the faces
 // behind the tile would cost four more cells and their logarithms, and tiles
 // at a shock cost several times the others, so there a segment is one tile.
+// The midpoints 0 .. 4 of such a tile belong to the tile before it too, and
+// either may evaluate one that the other does not need.  So that a fallback
+// there is counted once whatever the tiles, the left tile counts what it
+// evaluates, and this one what the left one does not: it needs the weights of
+// the faces -4 .. -1, that is the sensors of two more cells (CUT; the loads
+// and weights fill the same rounds of the workgroup as without them).
 #pragma once
 #include "em_device.h"
 #include "em_types.h"
@@ -30,12 +36,14 @@ namespace EM_VARIANT {
 // lanes then run along the cells and the rows of a pencil are contiguous
 // (with the pencils fast, as on strided axes, the loads along the axis would
 // hit the same banks 8 ways).
-template <class Real, int MODE, int T_, int P_, bool CF>
+// CUT: pencils may be cut into several segments.
+template <class Real, int MODE, int T_, int P_, bool CF, bool CUT>
 struct Tile {
     static constexpr int T = T_, P = P_;
     static constexpr bool HYB = MODE == MODE_HYBRID;
     static constexpr int HC = 10, HM = 5;  // slots taken over: cells, midpoints
-    static constexpr int C = T + HC, M = T + HM, TH = T + 1;
+    static constexpr int XC = HYB && CUT ? 2 : 0, XF = HYB && CUT ? 4 : 0;  // sensors and weights before slot 0
+    static constexpr int C = T + HC, M = T + HM, CS = C + XC, TH = T + 1 + XF;
     // a work item's slot and pencil: items [0, T P) are the tile's own slots
     // H .. H + T - 1, items [-H P, 0) the H slots before them
     template <int H>
@@ -52,12 +60,13 @@ struct Tile {
     }
     __device__ static __forceinline__ int at(int c, int p) { return CF ? p * C + c : c * P + p; }
     __device__ static __forceinline__ int mt(int m, int p) { return CF ? p * M + m : m * P + p; }
-    __device__ static __forceinline__ int tt(int f, int p) { return CF ? p * TH + f : f * P + p; }
+    __device__ static __forceinline__ int st(int c, int p) { return CF ? p * CS + c + XC : (c + XC) * P + p; }
+    __device__ static __forceinline__ int tt(int f, int p) { return CF ? p * TH + f + XF : (f + XF) * P + p; }
     Real sw[5][C * P];  // primitives
     Real sre[C * P];    // rho_e of each cell
     Real sm[5][M * P];  // midpoint fluxes; then the flux of face f in slot f - 1
     Real sf[5][P];      // flux of face 0
-    Real ss[2][HYB ? C * P : 1];
+    Real ss[2][HYB ? CS * P : 1];
     Real sth[HYB ? TH * P : 1];
 };
 
@@ -86,16 +95,17 @@ __device__ __forceinline__ void tile_faces(TL& L, int tid, bool first, int Tv, i
     auto& sm = L.sm;
     // ---- 2. hybrid blend weights (scheme.rs:171-183)
     if constexpr (HYB) {
-        for (int it = tid - P; it < T * P; it += NT) {
+        for (int it = tid - (1 + TL::XF) * P; it < T * P; it += NT) {
             int f, p;
-            TL::template item<1>(it, f, p);
-            if (p >= Pv || f > Tv) continue;
+            TL::template item<1 + TL::XF>(it, f, p);
+            f -= TL::XF;
+            if (p >= Pv || f > Tv || (f < 0 && s0 == 0)) continue;
             R r = R(0.0);
 #pragma unroll
             for (int k = 0; k < 2; ++k) {
                 R q[6];
 #pragma unroll
-                for (int j = 0; j < 6; ++j) q[j] = L.ss[k][TL::at(f + 2 + j, p)];
+                for (int j = 0; j < 6; ++j) q[j] = L.ss[k][TL::st(f + 2 + j, p)];
                 r = fmax(fmax(r, d4(q[0], q[1], q[2], q[3], q[4])), d4(q[1], q[2], q[3], q[4], q[5]));
             }
             R x = (r / tol - R(0.5)) / R(0.5);
@@ -131,9 +141,15 @@ __device__ __forceinline__ void tile_faces(TL& L, int tid, bool first, int Tv, i
 #pragma unroll
             for (int k = 0; k < 5; ++k) sm[k][TL::mt(m, p)] = f[k];
             if (fb) {
-                // global midpoint index; owned by one segment of the pencil
-                const int j = c0 - 3 + m;
-                if ((s0 == 0 || j >= s0) && (s1 == nD || j < s1)) atomicAdd(&scnt[1], 1u);
+                // counted by one segment of the pencil
+                const int j = c0 - 3 + m;  // global midpoint index
+                bool own = (s0 == 0 || j >= s0) && (s1 == nD || j < s1);
+                if constexpr (TL::XF > 0) {
+                    own = true;
+                    if (s0 > 0)
+                        for (int f = m - 4; f <= 0; ++f) own = own && !(L.sth[TL::tt(f, p)] > R(0.0));
+                }
+                if (own) atomicAdd(&scnt[1], 1u);
             }
         }
         __syncthreads();

@@ -87,7 +87,7 @@ __device__ __forceinline__ void ghost_state(const PassArgsT<Real>& a, long long 
 
 // LDS of a pass (declared by the kernels, passed to axis_segment)
 template <class Real, int MODE, int T, int P, bool CF, int NT>
-struct PassLds : Tile<Real, MODE, T, P, CF> {
+struct PassLds : Tile<Real, MODE, T, P, CF, true> {
     double sred[NT / 64 + 1];  // per-wave CFL rate (in double for the slot max)
     unsigned int scnt[3];
 };
@@ -97,7 +97,7 @@ struct PassLds : Tile<Real, MODE, T, P, CF> {
 // workgroup calls it; it returns uniformly).
 template <class Real, int D, int MODE, int T, int P, bool CF, int NT>
 __device__ __forceinline__ void axis_segment(const PassArgsT<Real>& a, int bid, PassLds<Real, MODE, T, P, CF, NT>& L) {
-    using TL = Tile<Real, MODE, T, P, CF>;
+    using TL = Tile<Real, MODE, T, P, CF, true>;
     constexpr bool HYB = MODE == MODE_HYBRID;
     auto& sw = L.sw;
     auto& sm = L.sm;
@@ -139,11 +139,12 @@ __device__ __forceinline__ void axis_segment(const PassArgsT<Real>& a, int bid, 
         const int Tv = min(T, s1 - c0);
         // ---- 1. load + primitives
 #pragma unroll 1
-        for (int it = tid - (first ? TL::HC * P : 0); it < T * P; it += NT) {
+        for (int it = tid - (first ? (TL::HC + TL::XC) * P : 0); it < T * P; it += NT) {
             int c, p;
-            TL::template item<TL::HC>(it, c, p);
+            TL::template item<TL::HC + TL::XC>(it, c, p);
+            c -= TL::XC;
             const int g = c0 - 5 + c;
-            if (p >= Pv || c >= Tv + TL::HC || g >= nD + 5) continue;
+            if (p >= Pv || c >= Tv + TL::HC || g >= nD + 5 || (c < 0 && c0 == 0)) continue;
             const long long pen = base + (long long)p * sF;
             Real u[5], w[5];
             if (g >= 0 && g < nD) {
@@ -155,15 +156,16 @@ __device__ __forceinline__ void axis_segment(const PassArgsT<Real>& a, int bid, 
             }
             Real v;
             to_prim_v(e, u, w, v);
+            if constexpr (HYB) {
+                // Euler::sensor, system.rs:409-413
+                L.ss[0][TL::st(c, p)] = log(fmax(w[0], Real(1e-300)));
+                L.ss[1][TL::st(c, p)] = log(fmax(w[4] + e.p_inf, Real(1e-300)));
+                if (c < 0) continue;  // the sensor alone
+            }
             const int q = TL::at(c, p);
 #pragma unroll
             for (int k = 0; k < 5; ++k) sw[k][q] = w[k];
             L.sre[q] = eos_rho_e_v(e, w[0], w[4], v);
-            if constexpr (HYB) {
-                // Euler::sensor, system.rs:409-413
-                L.ss[0][q] = log(fmax(w[0], Real(1e-300)));
-                L.ss[1][q] = log(fmax(w[4] + e.p_inf, Real(1e-300)));
-            }
         }
         if (active == 0) return;
         // the midpoints and the face flux taken over from the last tile

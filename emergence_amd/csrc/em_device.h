@@ -425,14 +425,13 @@ __device__ __forceinline__ double weno5_linear(double v0, double v1, double v2, 
 // left and right are 8 times the interpolated values.  top is raised to the
 // high word of the product of the three beta + eps, ok cleared where the last
 // quotient needs the general division: the caller falls back to
-// weno5z_interp unless ok and top below beta_max.  The weight sums reach
-// 2^1002 there (flat sub-stencils beside a jump of 2^183); where the product
-// of the two overflows (from a jump of about 2^62 on) or a weighted sum does,
-// the quotients come out infinite.  TINY: zero
-// fields and fields below 2^-200 are taken here as well (ahead of a front in
-// gas at rest the velocities fall off to denormals over many cells: a tenth
-// of all cells in a shock-bubble run), and infinite results clear ok; without
-// it they are left to the caller.  91 issue slots a side (a reciprocal counts
+// weno5z_interp unless ok, top below beta_max and both values finite.  The
+// weight sums reach 2^1002 there (flat sub-stencils beside a jump of 2^183);
+// where the product of the two overflows (from a jump of about 2^62 on) or a
+// weighted sum does, the values come out infinite.  TINY: zero fields and
+// fields below 2^-200 are taken here as well (ahead of a front in gas at rest
+// the velocities fall off to denormals over many cells: a tenth of all cells
+// in a shock-bubble run).  91 issue slots a side (a reciprocal counts
 // four) against about 125.
 template <bool TINY>
 __device__ __forceinline__ void weno5z_pair(const double v[6], double& left, double& right, unsigned& top, bool& ok) {
@@ -492,7 +491,6 @@ __device__ __forceinline__ void weno5z_pair(const double v[6], double& left, dou
             right = 8.0 * weno5_linear(v[5], v[4], v[3], v[2], v[1]);
         }
     }
-    if (TINY) fine = fine && fmax(fabs(left), fabs(right)) <= Mid<double>::huge;
     ok = ok && fine;
 }
 
@@ -573,15 +571,12 @@ __device__ __forceinline__ bool midpoint_flux_mid(const Eos& e, bool zero1, bool
     const double c2l = div_by(e.gamma * (wl[4] + e.p_inf) * vl * vl, vbl, rcp_volume(e, wl[0], vbl));
     const double c2r = div_by(e.gamma * (wr[4] + e.p_inf) * vr * vr, vbr, rcp_volume(e, wr[0], vbr));
     // all of [lo, hi]: high words order like positive values, a negative one
-    // or NaN is above them all; wl[0] and wr[0] are infinite or NaN where a
-    // value of the fields 0, 1 and 4 is
+    // or NaN is above them all
     const unsigned mn = min(min(min(top_word(rho), top_word(vb)), min(top_word(c2), top_word(wl[0]))),
                             min(min(min(top_word(wr[0]), top_word(vbl)), top_word(vbr)), min(top_word(c2l), top_word(c2r))));
     const unsigned mx = max(max(max(top_word(rho), top_word(vb)), max(top_word(c2), top_word(wl[0]))),
                             max(max(max(top_word(wr[0]), top_word(vbl)), top_word(vbr)), max(top_word(c2l), top_word(c2r))));
-    ok = ok && top < top_word(Mid<double>::beta_max) && mn >= top_word(Mid<double>::lo) &&
-         mx < top_word(Mid<double>::hi) && fmax(fabs(wl[un]), fabs(wr[un])) < Mid<double>::hi;
-    if (!ok) return false;
+    ok = ok && top < top_word(Mid<double>::beta_max) && mn >= top_word(Mid<double>::lo) && mx < top_word(Mid<double>::hi);
     double ql[5], qr[5];
 #pragma unroll
     for (int s = 0; s < 2; ++s) {
@@ -595,6 +590,9 @@ __device__ __forceinline__ bool midpoint_flux_mid(const Eos& e, bool zero1, bool
         const double a = (w[4] + e.gamma * e.p_inf) * (s ? vbr : vbl);
         q[4] = w[0] * (div_by(a, e.gamma - 1.0, e.rg) + e.q) + ke;
     }
+    // both energies are positive; below the bound the velocities are in range
+    // and no reconstruction is infinite
+    if (!(ok && ql[4] + qr[4] < Mid<double>::energy_max)) return false;
     double x;
     hllc_flux<D, true>(wl, wr, ql, qr, sqrt_mid(c2l, x), sqrt_mid(c2r, x), il, ir, f);
     return true;

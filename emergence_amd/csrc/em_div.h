@@ -26,6 +26,7 @@ struct Mid<double> {
     static constexpr double tiny = 0x1p-900;               // quotients and dividends below go the general way
     static constexpr double huge = 0x1p+800;
     static constexpr double beta_max = 0x1p+100;  // product of three WENO smoothness indicators
+    static constexpr double energy_max = 0x1p+300;  // total energies of a midpoint's two states
     static constexpr double margin = 1e-9;        // relative slack of clearly_admissible (rounding: about 1e-15)
 };
 template <>

@@ -62,7 +62,7 @@ static void pair_case(const double v[6], long long& taken) {
     unsigned top = 0;
     bool ok = true;
     weno5z_pair<true>(v, l, r, top, ok);
-    if (!ok || top >= top_word(Mid<double>::beta_max)) return;
+    if (!ok || top >= top_word(Mid<double>::beta_max) || !isfinite(l + r)) return;
     ++taken;
     const double a = weno5z_interp(v[0], v[1], v[2], v[3], v[4]), b = weno5z_interp(v[5], v[4], v[3], v[2], v[1]);
     if (!same(0.125 * l, a)) report("weno left", v, 6, 0.125 * l, a);

@@ -95,15 +95,15 @@ __device__ __forceinline__ void amr_item(const AmrPassArgsT<Real>& pa, long long
         for (int q = 0; q < 5; ++q) L.sw[q][TL::at(c, p)] = wv[q];
         L.sre[TL::at(c, p)] = eos_rho_e_v(e, wv[0], wv[4], v);
         if constexpr (HYB) {
-            L.ss[0][TL::st(c, p)] = log(fmax(wv[0], Real(1e-300)));
-            L.ss[1][TL::st(c, p)] = log(fmax(wv[4] + e.p_inf, Real(1e-300)));
+            L.ss[0][TL::at(c, p)] = log(fmax(wv[0], Real(1e-300)));
+            L.ss[1][TL::at(c, p)] = log(fmax(wv[4] + e.p_inf, Real(1e-300)));
         }
     }
     __syncthreads();
     // amr.rs:1254; formed in double from the device dt and rounded to Real
     const double lam = pa.ndim_pos > 0.0 ? pa.ndim_pos * dtv / (double)dx : 0.0;
     tile_faces<D, MODE, NT>(L, tid, true, B, Pv, 0, 0, B, B, e, Real(lam), pa.tol, a.bd[(D + 1) % 3] == 1,
-                            a.bd[(D + 2) % 3] == 1, n_shock, scnt, [] {});
+                            a.bd[(D + 2) % 3] == 1, n_shock, scnt, [](int, int, int) { return Real(0.0); }, [] {});
     // ---- residual and boundary face fluxes
     for (int it = tid; it < B * P; it += NT) {
         int c, p;

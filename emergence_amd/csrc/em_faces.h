@@ -22,9 +22,9 @@
 // The midpoints 0 .. 4 of such a tile belong to the tile before it too, and
 // either may evaluate one that the other does not need.  So that a fallback
 // there is counted once whatever the tiles, the left tile counts what it
-// evaluates, and this one what the left one does not: it needs the weights of
-// the faces -4 .. -1, that is the sensors of two more cells (CUT; the loads
-// and weights fill the same rounds of the workgroup as without them).
+// evaluates, and this one what the left one does not; the weights of the faces
+// -4 .. -1 that this takes are evaluated for such a fallback only (with every
+// tile's other weights they cost 3% of a Hybrid residual).
 #pragma once
 #include "em_device.h"
 #include "em_types.h"
@@ -37,13 +37,13 @@ namespace EM_VARIANT {
 // (with the pencils fast, as on strided axes, the loads along the axis would
 // hit the same banks 8 ways).
 // CUT: pencils may be cut into several segments.
-template <class Real, int MODE, int T_, int P_, bool CF, bool CUT>
+template <class Real, int MODE, int T_, int P_, bool CF, bool CUT_>
 struct Tile {
     static constexpr int T = T_, P = P_;
+    static constexpr bool CUT = CUT_;
     static constexpr bool HYB = MODE == MODE_HYBRID;
     static constexpr int HC = 10, HM = 5;  // slots taken over: cells, midpoints
-    static constexpr int XC = HYB && CUT ? 2 : 0, XF = HYB && CUT ? 4 : 0;  // sensors and weights before slot 0
-    static constexpr int C = T + HC, M = T + HM, CS = C + XC, TH = T + 1 + XF;
+    static constexpr int C = T + HC, M = T + HM, TH = T + 1;
     // a work item's slot and pencil: items [0, T P) are the tile's own slots
     // H .. H + T - 1, items [-H P, 0) the H slots before them
     template <int H>
@@ -60,18 +60,35 @@ struct Tile {
     }
     __device__ static __forceinline__ int at(int c, int p) { return CF ? p * C + c : c * P + p; }
     __device__ static __forceinline__ int mt(int m, int p) { return CF ? p * M + m : m * P + p; }
-    __device__ static __forceinline__ int st(int c, int p) { return CF ? p * CS + c + XC : (c + XC) * P + p; }
-    __device__ static __forceinline__ int tt(int f, int p) { return CF ? p * TH + f + XF : (f + XF) * P + p; }
+    __device__ static __forceinline__ int tt(int f, int p) { return CF ? p * TH + f : f * P + p; }
     Real sw[5][C * P];  // primitives
     Real sre[C * P];    // rho_e of each cell
     Real sm[5][M * P];  // midpoint fluxes; then the flux of face f in slot f - 1
     Real sf[5][P];      // flux of face 0
-    Real ss[2][HYB ? CS * P : 1];
+    Real ss[2][HYB ? C * P : 1];
     Real sth[HYB ? TH * P : 1];
 };
 
 // lanes of the wave that satisfy c (called where the wave is whole)
 __device__ __forceinline__ unsigned wave_count(bool c) { return (unsigned)__popcll(__ballot(c)); }
+
+// Blend weight of a face from the sensors k of the six cells around it, read
+// through ld(j, k)
+template <class R, class LD>
+__device__ __forceinline__ R blend_weight(R tol, LD&& ld) {
+    R r = R(0.0);
+#pragma unroll
+    for (int k = 0; k < 2; ++k) {
+        R q[6];
+#pragma unroll
+        for (int j = 0; j < 6; ++j) q[j] = ld(j, k);
+        r = fmax(fmax(r, d4(q[0], q[1], q[2], q[3], q[4])), d4(q[1], q[2], q[3], q[4], q[5]));
+    }
+    R x = (r / tol - R(0.5)) / R(0.5);
+    if (x < R(0.0)) x = R(0.0);
+    if (x > R(1.0)) x = R(1.0);
+    return isfinite(r) ? x * x * (R(3.0) - R(2.0) * x) : R(1.0);
+}
 
 // On entry (after a barrier): the tile's cells are in sw, sre and ss.  On
 // exit (after a barrier): the flux of face f = 1 .. Tv is sm[k][mt(f - 1, p)],
@@ -80,12 +97,14 @@ __device__ __forceinline__ unsigned wave_count(bool c) { return (unsigned)__popc
 // shock-path faces are counted per wave (a scalar register), fallbacks and
 // limited faces, which are few, in scnt[1] and scnt[2].  before_last() is
 // called once the faces are in registers, ahead of the last two barriers: the
-// place to issue the loads of the phase that follows.  zero1, zero2: the axes of the transverse velocities
-// (D+1) % 3 and (D+2) % 3 are inactive (see midpoint_flux_mid).
-template <int D, int MODE, int NT, class R, class TL, class PRE>
+// place to issue the loads of the phase that follows.  left_sensor(p, h, k) is
+// sensor k of the cell h - 2 before pencil p's tile (Hybrid, CUT, s0 > 0).
+// zero1, zero2: the axes of the transverse velocities (D+1) % 3 and (D+2) % 3
+// are inactive (see midpoint_flux_mid).
+template <int D, int MODE, int NT, class R, class TL, class SEN, class PRE>
 __device__ __forceinline__ void tile_faces(TL& L, int tid, bool first, int Tv, int Pv, int c0, int s0, int s1, int nD,
                                            const EosT<R>& e, R lam, R tol, bool zero1, bool zero2,
-                                           unsigned& n_shock, unsigned (&scnt)[3], PRE&& before_last) {
+                                           unsigned& n_shock, unsigned (&scnt)[3], SEN&& left_sensor, PRE&& before_last) {
     constexpr int T = TL::T, P = TL::P;
     constexpr bool HYB = MODE == MODE_HYBRID;
     constexpr bool CEN = MODE == MODE_CENTRAL;
@@ -95,23 +114,12 @@ __device__ __forceinline__ void tile_faces(TL& L, int tid, bool first, int Tv, i
     auto& sm = L.sm;
     // ---- 2. hybrid blend weights (scheme.rs:171-183)
     if constexpr (HYB) {
-        for (int it = tid - (1 + TL::XF) * P; it < T * P; it += NT) {
+        for (int it = tid - P; it < T * P; it += NT) {
             int f, p;
-            TL::template item<1 + TL::XF>(it, f, p);
-            f -= TL::XF;
-            if (p >= Pv || f > Tv || (f < 0 && s0 == 0)) continue;
-            R r = R(0.0);
-#pragma unroll
-            for (int k = 0; k < 2; ++k) {
-                R q[6];
-#pragma unroll
-                for (int j = 0; j < 6; ++j) q[j] = L.ss[k][TL::st(f + 2 + j, p)];
-                r = fmax(fmax(r, d4(q[0], q[1], q[2], q[3], q[4])), d4(q[1], q[2], q[3], q[4], q[5]));
-            }
-            R x = (r / tol - R(0.5)) / R(0.5);
-            if (x < R(0.0)) x = R(0.0);
-            if (x > R(1.0)) x = R(1.0);
-            L.sth[TL::tt(f, p)] = isfinite(r) ? x * x * (R(3.0) - R(2.0) * x) : R(1.0);
+            TL::template item<1>(it, f, p);
+            if (p >= Pv || f > Tv) continue;
+            L.sth[TL::tt(f, p)] =
+                blend_weight(tol, [&](int j, int k) { return L.ss[k][TL::at(f + 2 + j, p)]; });
         }
         __syncthreads();
     }
@@ -144,10 +152,25 @@ __device__ __forceinline__ void tile_faces(TL& L, int tid, bool first, int Tv, i
                 // counted by one segment of the pencil
                 const int j = c0 - 3 + m;  // global midpoint index
                 bool own = (s0 == 0 || j >= s0) && (s1 == nD || j < s1);
-                if constexpr (TL::XF > 0) {
-                    own = true;
-                    if (s0 > 0)
-                        for (int f = m - 4; f <= 0; ++f) own = own && !(L.sth[TL::tt(f, p)] > R(0.0));
+                if constexpr (HYB && TL::CUT) {
+                    own = s0 == 0 || m > 4 || !(L.sth[TL::tt(0, p)] > R(0.0));
+                    if (own && s0 > 0 && m < 4) {
+                        R x[2][2] = {};  // sensors of the cells -2 and -1
+#pragma unroll 1
+                        for (int i = 0; i < 4; ++i) {
+                            const R y = left_sensor(p, i & 1, i >> 1);
+                            x[0][0] = i == 0 ? y : x[0][0];
+                            x[1][0] = i == 1 ? y : x[1][0];
+                            x[0][1] = i == 2 ? y : x[0][1];
+                            x[1][1] = y;
+                        }
+#pragma unroll 1
+                        for (int f = m - 4; f < 0; ++f)
+                            own = own && !(blend_weight(tol, [&](int j, int k) {
+                                               const int c = f + 2 + j;
+                                               return c == -2 ? x[0][k] : c == -1 ? x[1][k] : L.ss[k][TL::at(c, p)];
+                                           }) > R(0.0));
+                    }
                 }
                 if (own) atomicAdd(&scnt[1], 1u);
             }

@@ -55,11 +55,13 @@ __global__ __launch_bounds__(256) void k_host_out(const Real* __restrict__ dev, 
 }
 
 // The buffer and the two transfers of one solver (not thread-safe, like its
-// handle).  Both leave the stream idle: the host array is free on return.
+// handle).  Both leave the stream idle, also on an error: the host array is
+// free on return.
 template <int NV>
 struct HostIo {
     double* buf = nullptr;
-    long long cells = 0;  // capacity
+    long long cells = 0;           // capacity
+    size_t limit = kHostIoBytes;  // of the buffer
 
     HostIo() = default;
     HostIo(const HostIo&) = delete;
@@ -67,11 +69,15 @@ struct HostIo {
         if (buf) (void)hipFree(buf);
     }
     hipError_t reserve(const HostLayout& h) {
-        const long long want = std::min<long long>(h.len, (long long)(kHostIoBytes / (8 * NV)));
+        const long long want = std::min<long long>(h.len, (long long)(limit / (8 * NV)));
         if (cells >= want) return hipSuccess;
         const hipError_t e = hipMalloc(&buf, sizeof(double) * NV * want);
         if (e == hipSuccess) cells = want;
         return e;
+    }
+    static hipError_t finish(hipError_t e, hipStream_t s) {
+        const hipError_t f = hipStreamSynchronize(s);
+        return e == hipSuccess ? f : e;
     }
     template <class Real>
     hipError_t in(const HostLayout& h, const double* host, Real* dev, hipStream_t s) {
@@ -84,7 +90,7 @@ struct HostIo {
                                dev);
             e = hipGetLastError();
         }
-        return e == hipSuccess ? hipStreamSynchronize(s) : e;
+        return finish(e, s);
     }
     template <class Real>
     hipError_t out(const HostLayout& h, const Real* dev, bool padded, double* host, hipStream_t s) {
@@ -97,7 +103,7 @@ struct HostIo {
             if (e == hipSuccess)
                 e = hipMemcpyAsync(host + q0 * NV, buf, sizeof(double) * NV * cnt, hipMemcpyDeviceToHost, s);
         }
-        return e == hipSuccess ? hipStreamSynchronize(s) : e;
+        return finish(e, s);
     }
 };
 

@@ -139,12 +139,11 @@ __device__ __forceinline__ void axis_segment(const PassArgsT<Real>& a, int bid, 
         const int Tv = min(T, s1 - c0);
         // ---- 1. load + primitives
 #pragma unroll 1
-        for (int it = tid - (first ? (TL::HC + TL::XC) * P : 0); it < T * P; it += NT) {
+        for (int it = tid - (first ? TL::HC * P : 0); it < T * P; it += NT) {
             int c, p;
-            TL::template item<TL::HC + TL::XC>(it, c, p);
-            c -= TL::XC;
+            TL::template item<TL::HC>(it, c, p);
             const int g = c0 - 5 + c;
-            if (p >= Pv || c >= Tv + TL::HC || g >= nD + 5 || (c < 0 && c0 == 0)) continue;
+            if (p >= Pv || c >= Tv + TL::HC || g >= nD + 5) continue;
             const long long pen = base + (long long)p * sF;
             Real u[5], w[5];
             if (g >= 0 && g < nD) {
@@ -156,16 +155,15 @@ __device__ __forceinline__ void axis_segment(const PassArgsT<Real>& a, int bid, 
             }
             Real v;
             to_prim_v(e, u, w, v);
-            if constexpr (HYB) {
-                // Euler::sensor, system.rs:409-413
-                L.ss[0][TL::st(c, p)] = log(fmax(w[0], Real(1e-300)));
-                L.ss[1][TL::st(c, p)] = log(fmax(w[4] + e.p_inf, Real(1e-300)));
-                if (c < 0) continue;  // the sensor alone
-            }
             const int q = TL::at(c, p);
 #pragma unroll
             for (int k = 0; k < 5; ++k) sw[k][q] = w[k];
             L.sre[q] = eos_rho_e_v(e, w[0], w[4], v);
+            if constexpr (HYB) {
+                // Euler::sensor, system.rs:409-413
+                L.ss[0][q] = log(fmax(w[0], Real(1e-300)));
+                L.ss[1][q] = log(fmax(w[4] + e.p_inf, Real(1e-300)));
+            }
         }
         if (active == 0) return;
         // the midpoints and the face flux taken over from the last tile
@@ -188,7 +186,16 @@ __device__ __forceinline__ void axis_segment(const PassArgsT<Real>& a, int bid, 
         const long long idx = base + (long long)p * sF + (long long)(c0 + c) * sD;
         Real r[5], u0[5], us[5];
         tile_faces<D, MODE, NT>(L, tid, first, Tv, Pv, c0, s0, s1, nD, e, lam, a.tol, !a.active[(D + 1) % 3],
-                                !a.active[(D + 2) % 3], n_shock, scnt, [&] {
+                                !a.active[(D + 2) % 3], n_shock, scnt,
+                                [&](int p, int h, int k) {
+                                    Real u[5], w[5];
+                                    const long long i = base + (long long)p * sF + (long long)(c0 - 7 + h) * sD;
+#pragma unroll
+                                    for (int q = 0; q < 5; ++q) u[q] = a.U[q * nc + i];
+                                    to_prim(e, u, w);
+                                    return log(fmax(k ? w[4] + e.p_inf : w[0], Real(1e-300)));
+                                },
+                                [&] {
 #pragma unroll
                                     for (int k = 0; k < 5; ++k) {
                                         r[k] = a.first || !mine ? Real(0.0) : a.R[k * nc + idx];

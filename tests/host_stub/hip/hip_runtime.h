@@ -8,6 +8,7 @@
 #pragma once
 #include <cmath>
 #include <cstdint>
+#include <cstdlib>
 #include <cstring>
 
 #define __device__
@@ -76,3 +77,55 @@ template <class T>
 inline T min(T a, T b) {
     return a < b ? a : b;
 }
+
+// ---- the runtime calls of em_hostio.h: device memory is host memory, a
+// kernel launch runs its threads in turn
+typedef int hipError_t;
+typedef void* hipStream_t;
+constexpr hipError_t hipSuccess = 0, hipErrorOutOfMemory = 2, hipErrorUnknown = 999;
+enum { hipMemcpyHostToDevice = 1, hipMemcpyDeviceToHost = 2 };
+struct dim3 {
+    unsigned x;
+    explicit dim3(unsigned v) : x(v) {}
+};
+inline dim3 blockIdx(0), threadIdx(0);
+// what the tests watch and force
+struct StubState {
+    size_t malloc_limit = (size_t)-1;  // larger requests fail
+    int fail_copy = -1;                // the copy of this index fails
+    int copies = 0, mallocs = 0, frees = 0;
+    bool pending = false;              // work queued since the last synchronisation
+    size_t bytes = 0;                  // copied
+};
+inline StubState stub;
+template <class T>
+inline hipError_t hipMalloc(T** p, size_t n) {
+    if (n > stub.malloc_limit) return hipErrorOutOfMemory;
+    stub.mallocs++;
+    *p = (T*)std::malloc(n);
+    return hipSuccess;
+}
+inline hipError_t hipFree(void* p) {
+    stub.frees++;
+    std::free(p);
+    return hipSuccess;
+}
+inline hipError_t hipMemcpyAsync(void* d, const void* s, size_t n, int, hipStream_t) {
+    if (stub.copies++ == stub.fail_copy) return hipErrorUnknown;
+    std::memcpy(d, s, n);
+    stub.bytes += n;
+    stub.pending = true;
+    return hipSuccess;
+}
+inline hipError_t hipStreamSynchronize(hipStream_t) {
+    stub.pending = false;
+    return hipSuccess;
+}
+inline hipError_t hipGetLastError() { return hipSuccess; }
+template <class K, class... A>
+inline void stub_launch(K k, dim3 grid, dim3 block, A... a) {
+    for (blockIdx.x = 0; blockIdx.x < grid.x; ++blockIdx.x)
+        for (threadIdx.x = 0; threadIdx.x < block.x; ++threadIdx.x) k(a...);
+    stub.pending = true;
+}
+#define hipLaunchKernelGGL(k, grid, block, lds, stream, ...) stub_launch(k, grid, block, __VA_ARGS__)

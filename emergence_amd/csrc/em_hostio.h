@@ -79,10 +79,6 @@ struct HostIo {
         const hipError_t f = hipStreamSynchronize(s);
         return e == hipSuccess ? f : e;
     }
-    static hipError_t finish(hipError_t e, hipStream_t s) {
-        const hipError_t f = hipStreamSynchronize(s);
-        return e == hipSuccess ? f : e;
-    }
     template <class Real>
     hipError_t in(const HostLayout& h, const double* host, Real* dev, hipStream_t s) {
         hipError_t e = reserve(h);

@@ -1,20 +1,34 @@
 // Conversion between a solver's device layout (interior cells, variable-major
 // planes of ncell values) and the host layout of the C ABI (ghost-padded
-// cells, NV doubles each), on the device: the host copies bytes only.
+// cells, NV doubles each).
 //
-// Bound by the host link (17 to 28 GB/s for pageable memory here; the kernels
-// run at several TB/s).  The strided single-thread loops this replaces took
-// about 25 ms each way for a 128^3 state (110 MB in the host layout), against
-// 4 to 7 ms of copying.  Large arrays go through a buffer of at most
-// kHostIoBytes in pieces, so the extra device memory is bounded.
+// Large states are converted on the device, so that the host copies bytes
+// only: bound by the host link (17 to 28 GB/s for pageable memory here; the
+// kernels run at several TB/s).  The strided single-thread loops took about
+// 25 ms each way for a 128^3 state (110 MB in the host layout), the copies
+// take 4 to 7 ms.  Large arrays go through a buffer of at most kHostIoBytes in
+// pieces, so the extra device memory is bounded.
+//
+// The device path moves the ghosts over the link too and needs a kernel more.
+// States that fit the host's caches are converted in a loop on the host where
+// that is faster (HostIo::..._on_host): small ones, and thin meshes, whose
+// padded array is many times the interior.  It also serves where the buffer
+// cannot be had.  In microseconds, host loop / device:
+//   in:  33x47 15/27, 64x64 23/31, 16^3 19/53, 1000x4x4 61/310,
+//        2x200x300 328/1291, 45x64x50 341/326, 512^2 833/339
+//   out (seven variables): 64x48 25/36, 40x30x20 179/242, 1000x4x4 180/832
 #pragma once
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <vector>
 
 namespace em {
 
 constexpr size_t kHostIoBytes = 256u << 20;
+// bytes read and written up to which the host loops stay in the caches (12 to
+// 17 GB/s; 3.5 GB/s at 80 MB)
+constexpr double kHostLoopBytes = 16e6;
 
 // Padded extents and ghost offsets of a mesh (int: a padded plane index fits)
 struct HostLayout {
@@ -22,6 +36,12 @@ struct HostLayout {
     int m1, m2;            // padded extents of the inner axes
     int g0, g1, g2;        // ghost offsets
     long long ncell, len;  // interior and padded cells
+    // f(padded index, interior index) of the first cell of every interior row
+    template <class F>
+    void for_rows(F&& f) const {
+        for (long long i = 0; i < n0; ++i)
+            for (long long j = 0; j < n1; ++j) f(((i + g0) * m1 + (j + g1)) * m2 + g2, (i * n1 + j) * n2);
+    }
     // interior index of padded cell q, or -1
     __device__ __forceinline__ long long interior(long long q) const {
         const long long i = q / ((long long)m1 * m2) - g0, j = (q / m2) % m1 - g1, k = q % m2 - g2;
@@ -68,20 +88,95 @@ struct HostIo {
     ~HostIo() {
         if (buf) (void)hipFree(buf);
     }
-    hipError_t reserve(const HostLayout& h) {
-        const long long want = std::min<long long>(h.len, (long long)(limit / (8 * NV)));
-        if (cells >= want) return hipSuccess;
-        const hipError_t e = hipMalloc(&buf, sizeof(double) * NV * want);
-        if (e == hipSuccess) cells = want;
-        return e;
-    }
     static hipError_t finish(hipError_t e, hipStream_t s) {
         const hipError_t f = hipStreamSynchronize(s);
         return e == hipSuccess ? f : e;
     }
+    // false: no memory for the buffer
+    bool reserve(const HostLayout& h) {
+        const long long want = std::min<long long>(h.len, (long long)(limit / (8 * NV)));
+        if (cells >= want) return true;
+        if (buf) (void)hipFree(buf);
+        buf = nullptr;
+        cells = 0;
+        if (hipMalloc(&buf, sizeof(double) * NV * want) != hipSuccess) {
+            (void)hipGetLastError();
+            buf = nullptr;
+            return false;
+        }
+        cells = want;
+        return true;
+    }
+    // Which side converts, by the time of either (microseconds, bytes per
+    // microsecond): a loop over the interior at 16 GB/s (23 in float, half
+    // the bytes to write and copy) against the whole padded array at 30 GB/s
+    // and a kernel
+    template <class Real>
+    static bool in_on_host(const HostLayout& h) {
+        const double ib = 8.0 * NV * h.ncell, pb = 8.0 * NV * h.len;
+        return ib * (1.0 + sizeof(Real) / 8.0) <= kHostLoopBytes &&
+               10.0 + ib / (sizeof(Real) == 4 ? 23e3 : 16e3) < 20.0 + pb / 30e3;
+    }
+    // out: interior planes are copied at 17 GB/s and scattered (8.2 together,
+    // 15 in float) into zeros, or the padded array copied at 17.5; padded
+    // planes of doubles lose the transposition at 37 GB/s but save a kernel; in
+    // float they are half the bytes, which weighs more as long as the staging
+    // array is not mapped anew for each call (above 32 MB)
+    template <class Real>
+    static bool out_on_host(const HostLayout& h, bool padded) {
+        const double ib = 8.0 * NV * h.ncell, pb = 8.0 * NV * h.len;
+        if (padded)
+            return sizeof(Real) == 4 ? pb <= 64e6 && pb / 27e3 < 5.0 + pb / 17.5e3 : pb / 11.9e3 < 5.0 + pb / 17.5e3;
+        return ib * (1.0 + sizeof(Real) / 8.0) <= kHostLoopBytes &&
+               10.0 + ib / (sizeof(Real) == 4 ? 15e3 : 8.2e3) + pb / 200e3 < 24.0 + pb / 17.5e3;
+    }
+    template <class Real>
+    hipError_t in_by_host(const HostLayout& h, const double* host, Real* dev, hipStream_t s) {
+        // a cleared array for each call: the clearing brings its lines into the
+        // caches (an uncleared or a kept one took up to twice the time)
+        std::vector<Real> t(NV * h.ncell);
+        Real* const p = t.data();
+        const long long nc = h.ncell, n2 = h.n2;
+        h.for_rows([=](long long q, long long c) {
+            const double* u = host + q * NV;
+            for (long long k = 0; k < n2; ++k, u += NV)
+                for (int v = 0; v < NV; ++v) p[v * nc + c + k] = Real(u[v]);
+        });
+        return finish(hipMemcpyAsync(dev, t.data(), sizeof(Real) * NV * h.ncell, hipMemcpyHostToDevice, s), s);
+    }
+    template <class Real>
+    hipError_t out_by_host(const HostLayout& h, const Real* dev, bool padded, double* host, hipStream_t s) {
+        const long long plane = padded ? h.len : h.ncell;
+        std::vector<Real> t(NV * plane);
+        const hipError_t e = finish(hipMemcpyAsync(t.data(), dev, sizeof(Real) * NV * plane, hipMemcpyDeviceToHost, s), s);
+        if (e != hipSuccess) return e;
+        if (padded) {
+            for (long long q = 0; q < h.len; ++q)
+                for (int v = 0; v < NV; ++v) host[q * NV + v] = (double)t[v * plane + q];
+            return e;
+        }
+        std::fill(host, host + NV * h.len, 0.0);
+        const Real* const p = t.data();
+        const long long n2 = h.n2;
+        h.for_rows([=](long long q, long long c) {
+            double* u = host + q * NV;
+            for (long long k = 0; k < n2; ++k, u += NV)
+                for (int v = 0; v < NV; ++v) u[v] = (double)p[v * plane + c + k];
+        });
+        return e;
+    }
     template <class Real>
     hipError_t in(const HostLayout& h, const double* host, Real* dev, hipStream_t s) {
-        hipError_t e = reserve(h);
+        return in_on_host<Real>(h) ? in_by_host(h, host, dev, s) : in_by_device(h, host, dev, s);
+    }
+    template <class Real>
+    hipError_t out(const HostLayout& h, const Real* dev, bool padded, double* host, hipStream_t s) {
+        return out_on_host<Real>(h, padded) ? out_by_host(h, dev, padded, host, s) : out_by_device(h, dev, padded, host, s);
+    }
+    template <class Real>
+    hipError_t in_by_device(const HostLayout& h, const double* host, Real* dev, hipStream_t s) {
+        if (!reserve(h)) return in_by_host(h, host, dev, s);
+        hipError_t e = hipSuccess;
         for (long long q0 = 0; e == hipSuccess && q0 < h.len; q0 += cells) {
             const long long cnt = std::min(cells, h.len - q0);
             e = hipMemcpyAsync(buf, host + q0 * NV, sizeof(double) * NV * cnt, hipMemcpyHostToDevice, s);
@@ -93,8 +188,9 @@ struct HostIo {
         return finish(e, s);
     }
     template <class Real>
-    hipError_t out(const HostLayout& h, const Real* dev, bool padded, double* host, hipStream_t s) {
-        hipError_t e = reserve(h);
+    hipError_t out_by_device(const HostLayout& h, const Real* dev, bool padded, double* host, hipStream_t s) {
+        if (!reserve(h)) return out_by_host(h, dev, padded, host, s);
+        hipError_t e = hipSuccess;
         for (long long q0 = 0; e == hipSuccess && q0 < h.len; q0 += cells) {
             const long long cnt = std::min(cells, h.len - q0);
             hipLaunchKernelGGL((k_host_out<NV, Real>), dim3((unsigned)((cnt + 255) / 256)), dim3(256), 0, s, dev, h,

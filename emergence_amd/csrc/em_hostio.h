@@ -21,6 +21,7 @@
 #include <hip/hip_runtime.h>
 
 #include <algorithm>
+#include <mutex>
 #include <vector>
 
 namespace em {
@@ -74,11 +75,12 @@ __global__ __launch_bounds__(256) void k_host_out(const Real* __restrict__ dev, 
     for (int v = 0; v < NV; ++v) io[t * NV + v] = c < 0 ? 0.0 : (double)dev[v * plane + c];
 }
 
-// The buffer and the two transfers of one solver (not thread-safe, like its
-// handle).  Both leave the stream idle, also on an error: the host array is
+// The buffer and the two transfers of one solver, or of an ensemble's instances
+// (whose transfers may come from several threads).  Both leave the stream idle, also on an error: the host array is
 // free on return.
 template <int NV>
 struct HostIo {
+    std::mutex lock;  // of the buffer
     double* buf = nullptr;
     long long cells = 0;           // capacity
     size_t limit = kHostIoBytes;  // of the buffer
@@ -175,6 +177,7 @@ struct HostIo {
     }
     template <class Real>
     hipError_t in_by_device(const HostLayout& h, const double* host, Real* dev, hipStream_t s) {
+        const std::lock_guard<std::mutex> hold(lock);
         if (!reserve(h)) return in_by_host(h, host, dev, s);
         hipError_t e = hipSuccess;
         for (long long q0 = 0; e == hipSuccess && q0 < h.len; q0 += cells) {
@@ -189,6 +192,7 @@ struct HostIo {
     }
     template <class Real>
     hipError_t out_by_device(const HostLayout& h, const Real* dev, bool padded, double* host, hipStream_t s) {
+        const std::lock_guard<std::mutex> hold(lock);
         if (!reserve(h)) return out_by_host(h, dev, padded, host, s);
         hipError_t e = hipSuccess;
         for (long long q0 = 0; e == hipSuccess && q0 < h.len; q0 += cells) {

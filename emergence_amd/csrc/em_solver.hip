@@ -364,7 +364,8 @@ struct SolverCore : Grid {
     Real* U[3] = {nullptr, nullptr, nullptr};  // U^n, stage 1, stage 2
     Real* R = nullptr;
     Real* pad = nullptr;
-    HostIo<5> io;  // conversion buffer of upload, download and the host-array entry points
+    HostIo<5> own_io;  // conversion buffer of upload, download and the host-array entry points
+    HostIo<5>* io = &own_io;  // (an ensemble's instances share one)
     Real* bcdev = nullptr;  // [3][2][5] boundary states for the ghost sweep
     double* dt_hist = nullptr;  // device dt history of a CFL-driven forward run
     int64_t dt_hist_cap = 0;
@@ -411,7 +412,7 @@ struct SolverCore : Grid {
     HostLayout host_layout() const { return HostLayout{n[0], n[1], n[2], m(1), m(2), g(0), g(1), g(2), ncell, len()}; }
 
     void upload(const double* u) {
-        HIPCHK(io.in(host_layout(), u, U[0], stream));
+        HIPCHK(io->in(host_layout(), u, U[0], stream));
         rate_valid = false;
     }
 
@@ -452,7 +453,7 @@ struct SolverCore : Grid {
 
     void download(double* u) {
         fill_pad();
-        HIPCHK(io.out(host_layout(), pad, true, u, stream));
+        HIPCHK(io->out(host_layout(), pad, true, u, stream));
     }
 
     PassArgsT<Real> pass_args(int d) const { return Grid::pass_args_t<Real>(d, sc); }
@@ -558,7 +559,7 @@ struct SolverCore : Grid {
         reset_run(0.0);
         stage(U[0], nullptr, 0, false, 1, stage_dt, nullptr);
         Scalars after = read_scalars();
-        HIPCHK(io.out(host_layout(), R, false, out, stream));
+        HIPCHK(io->out(host_layout(), R, false, out, stream));
         if (stats) {
             stats[0] = faces_per_stage();
             for (int q = 0; q < 3; ++q) stats[1 + q] = after.counters[q] - before.counters[q];
@@ -828,8 +829,8 @@ struct Solver : SolverCore<double> {
         }
     }
 
-    void host_to_soa(const double* u, double* dev) { HIPCHK(io.in(host_layout(), u, dev, stream)); }
-    void soa_to_host(const double* dev, double* u) { HIPCHK(io.out(host_layout(), dev, false, u, stream)); }
+    void host_to_soa(const double* u, double* dev) { HIPCHK(io->in(host_layout(), u, dev, stream)); }
+    void soa_to_host(const double* dev, double* u) { HIPCHK(io->out(host_layout(), dev, false, u, stream)); }
 
     void ensure_adjbuf() {
         if (!adjbuf) HIPCHK(hipMalloc(&adjbuf, sizeof(double) * 20 * ncell));
@@ -1145,6 +1146,7 @@ __global__ void k_ens_copy(const CopyTask* __restrict__ t) {
 // one HIP graph; the adjoint launches each instance's VJP (adj_pass).
 struct Ensemble {
     std::vector<Solver*> in;
+    HostIo<5> io;  // of all instances, which transfer one after another
     int n = 0;
     int mode, cfg = 4, precise = 1;
     bool batched = true;
@@ -1187,6 +1189,7 @@ struct Ensemble {
         try {
             for (int i = 0; i < n; ++i) {
                 in.push_back(new Solver(nn + 3 * i, lo + 3 * i, hi + 3 * i, ng, e, bk, bs, mode_, pos, cfl_, tol, 0.0));
+                in.back()->io = &io;
                 in.back()->upload(u[i]);
             }
         } catch (...) {

@@ -51,3 +51,37 @@ def test_fiveeq_upload_and_download(real, n):
     d = g.download()
     assert np.array_equal(_interior(d, n), want)
     assert d.sum() == _interior(d, n).sum() or np.isclose(d.sum(), _interior(d, n).sum(), rtol=1e-12)
+
+
+def _free_bytes():
+    import ctypes as C
+
+    from emergence_amd import DeviceArray
+
+    free, total = C.c_size_t(), C.c_size_t()
+    assert DeviceArray._rt().hipMemGetInfo(C.byref(free), C.byref(total)) == 0
+    return free.value
+
+
+def test_an_ensemble_holds_one_conversion_buffer():
+    """Its instances' transfers, also from several threads, go through one
+    buffer (each its own: 129 MB here)."""
+    from concurrent.futures import ThreadPoolExecutor
+
+    import emergence_amd as em
+
+    sizes = [(512, 512, 1)] * 11 + [(300, 400, 1)]  # the largest comes first and again after smaller ones
+    rng = np.random.default_rng(1)
+    us = [1.0 + 0.1 * rng.random((n[0] + 12, n[1] + 12, 1, 5)) + 2.0 * (np.arange(5) == 4) for n in sizes]
+    em.HipSolver((64, 64, 1), (0, 0, 0), (1, 1, 1), us[0][:76, :76], mode="central").rhs(1e-3)  # context and code
+    before = _free_bytes()
+    e = em.HipEnsemble(sizes, us, mode="central")
+    used = before - _free_bytes()
+    states = 4 * 40 * sum(n[0] * n[1] for n in sizes)
+    assert used < states + 80e6, (used, states)
+    with ThreadPoolExecutor(4) as pool:
+        for _ in range(3):
+            list(pool.map(lambda i: e.upload(i, (i + 2.0) * us[i]), range(len(sizes))))
+            got = list(pool.map(e.download, range(len(sizes))))
+            for i, n in enumerate(sizes):
+                assert np.array_equal(_interior(got[i], n), (i + 2.0) * _interior(us[i], n)), i

@@ -336,10 +336,18 @@ struct Grid {
     // midpoint (512^2: 29-33 us against 31-34); and a few one-wave tiles for
     // the smallest grids, whose time is one tile's latency (64^2 Hybrid: 16
     // us against 16-21).
-    int default_cfg(int d) const {
+    // FP32: a tile's work is smaller and more of it divergent (the general
+    // divisions, limited faces and fallbacks of rough states), so the line is
+    // higher and the contiguous axis takes one-wave tiles below it (121x136x103
+    // Weno, outflow: 156, 177 and 171 us an axis against 210, 209 and 218 in
+    // 32-cell tiles; Hybrid z axis 189 against 281 in 27-cell tiles; 160^3
+    // Weno, 19,200 tiles: 200-228 us in 32-cell tiles against 221-251).  Pencils
+    // of one tile stay with the 27-cell shape (300x20x20, z: 23 against 28 us).
+    int default_cfg(int d, bool f32 = false) const {
         const int f = active(d == 2 ? 1 : 2) ? (d == 2 ? 1 : 2) : (d == 0 ? 1 : 0);
         const long long tiles = (n[d] + 26) / 27 * ((n[f] + 7) / 8) * (ncell / n[d] / n[f]);
         if (tiles < 256) return 6;
+        if (f32 && mode != MODE_CENTRAL && tiles < 12000) return stride[d] == 1 && n[d] > 27 ? 7 : 3;
         if (mode == MODE_HYBRID) return 3;
         return tiles < 4096 ? (stride[d] == 1 ? 4 : 3) : 0;
     }
@@ -379,6 +387,7 @@ struct SolverCore : Grid {
     SolverCore(const int64_t nn[3], const double lo_[3], const double hi[3], int ng_, const double e[4],
                const int32_t bk[6], const double bs[30], int mode_, int pos, double cfl_, double tol_, double t0)
         : Grid(nn, lo_, hi, ng_, e, bk, bs, mode_, pos, cfl_, tol_) {
+        for (int d = 0; d < 3; ++d) cfg[d] = default_cfg(d, sizeof(Real) == 4);
         HIPCHK(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
         for (int b = 0; b < 3; ++b) HIPCHK(hipMalloc(&U[b], sizeof(Real) * 5 * ncell));
         HIPCHK(hipMalloc(&R, sizeof(Real) * 5 * ncell));

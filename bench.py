@@ -43,8 +43,9 @@ CFL = 0.5
 # 3,500 FLOP per cell per RK stage in 3-D, i.e. 3,500/3 per cell per axis pass.
 # tile shapes of the axis pass (T cells, P pencils, threads) by cfg id, as
 # the library's table
-TILE_SHAPES = [(32, 16, 640), (64, 8, 576), (128, 4, 576), (256, 2, 576), (27, 8, 256), (59, 4, 256), (59, 8, 512),
-               (27, 16, 512), (123, 4, 512), (59, 16, 1024)]
+TILE_SHAPES = [(32, 8, 256), (64, 8, 512), (59, 1, 64), (27, 2, 64), (27, 8, 256), (59, 4, 256), (27, 4, 128),
+               (16, 16, 256), (123, 4, 512), (16, 4, 64)]
+DEFAULT_TILES = {"weno": [0, 0, 0], "hybrid": [4, 4, 4]}  # the library's choice at 256^3
 FLOP_PER_CELL_STAGE = 3500.0
 FLOP_PER_CELL_STAGE_CENTRAL = 1600.0  # KEEP-PE central flux on every face, 3-D
 BYTES_PER_CELL_STAGE = 120.0  # read U^(s), read U^n, write U^(s+1) (5 x f64 each)
@@ -65,7 +66,7 @@ def parse():
     ap.add_argument("--cpu-repeats", type=int, default=4, help="CPU-baseline repeats (median)")
     ap.add_argument("--no-autotune", action="store_true", help="keep the default tile shapes (short profiled runs)")
     ap.add_argument("--tiles", type=str, default=None,
-                    help="fixed Weno tile shapes per axis, e.g. 6,6,5 (indices into TILE_SHAPES; no autotuning)")
+                    help="fixed Weno tile shapes per axis, e.g. 0,0,9 (indices into TILE_SHAPES; no autotuning)")
     ap.add_argument("--hybrid-tiles", type=str, default=None, help="fixed Hybrid tile shapes per axis")
     ap.add_argument("--no-f32", action="store_true", help="skip the FP32 lines (256^3 Euler, FiveEq probe, AMR)")
     ap.add_argument("--f32-tiles", type=str, default=None, help="fixed FP32 tile shapes per axis")
@@ -587,7 +588,8 @@ def profiled_traffic(variant, mode, d, shape):
     path = os.path.join(ROOT, "profiles", "axis_pass_256cubed.md")
     if not os.path.exists(path):
         return None
-    sig = f"`em::{variant}::axis_pass<{d}, {mode}, {shape[0]}, {shape[1]}, {shape[2]}>`"
+    # the last axis is the contiguous one, whose kernels keep a pencil's cells together in LDS
+    sig = f"`em::{variant}::axis_pass<{d}, {mode}, {shape[0]}, {shape[1]}, {'true' if d == 2 else 'false'}, {shape[2]}>`"
     for line in open(path):
         cells = [c.strip() for c in line.split("|")]
         # | kernel | read requests | read | write | read + write | algorithmic | ratio |
@@ -807,7 +809,7 @@ def hybrid_bench(em, args, n, u):
         "roofline": {"bound": "mfma", "roof": "fp64-valu", "kernel": f"axis_pass d={dom}", "achieved": achieved / 1e12,
                      "peak": PEAK_FP64 / 1e12, "unit": "TFLOP/s", "frac": achieved / PEAK_FP64,
                      "traffic": profiled_traffic("fast" if args.fast else "precise", 0, dom,
-                                                 TILE_SHAPES[(tiles or [6, 6, 6])[dom]]),
+                                                 TILE_SHAPES[(tiles or DEFAULT_TILES["hybrid"])[dom]]),
                      "flop_per_cell_stage": flop, "hbm_fraction": value * BYTES_PER_CELL_STAGE / PEAK_HBM},
     }
 
@@ -885,7 +887,7 @@ def main():
             "peak": PEAK_FP64 / 1e12,
             "unit": "TFLOP/s",
             "frac": achieved / PEAK_FP64,
-            "traffic": profiled_traffic("fast" if args.fast else "precise", 1, dom, TILE_SHAPES[(tiles or [6, 6, 6])[dom]]),
+            "traffic": profiled_traffic("fast" if args.fast else "precise", 1, dom, TILE_SHAPES[(tiles or DEFAULT_TILES["weno"])[dom]]),
             "hbm_fraction": value * BYTES_PER_CELL_STAGE / PEAK_HBM,
             "fp64_fraction": value * FLOP_PER_CELL_STAGE / PEAK_FP64,
         },

@@ -7,12 +7,16 @@
 
 namespace em {
 
-// Tile shapes (cells along the axis x pencils, threads); index = cfg id.  A
-// strided pass reads P neighbouring cells of the innermost axis.  One thread
-// per cell (T P == NT) suits segments of many tiles, one per midpoint
-// ((T + 5) P == NT) those of one tile.
-constexpr TileCfg kTileCfgs[] = {{32, 8, 256}, {16, 16, 256}, {64, 8, 512}, {27, 8, 256}, {59, 4, 256},
-                                 {27, 4, 128}, {27, 2, 64}, {59, 1, 64}, {16, 4, 64}, {123, 4, 512}};
+// Tile shapes (cells along the axis x pencils, threads); index = cfg id, part
+// of the interface (em_solver_set_tiles: a program may have stored one, so a
+// changed table keeps the surviving shapes' indices and puts under the others
+// shapes that are no slower than what stood there).  A strided pass reads P
+// neighbouring cells of the innermost axis.  One thread per cell (T P == NT)
+// suits segments of many tiles, one per midpoint ((T + 5) P == NT) those of
+// one tile.
+constexpr TileCfg kTileCfgs[] = {{32, 8, 256}, {64, 8, 512}, {59, 1, 64}, {27, 2, 64}, {27, 8, 256},
+                                 {59, 4, 256}, {27, 4, 128}, {16, 16, 256}, {123, 4, 512}, {16, 4, 64}};
+enum : int { TILE_32x8 = 0, TILE_59x1 = 2, TILE_27x2 = 3, TILE_27x8 = 4, TILE_59x4 = 5 };
 constexpr int kNumTileCfgs = 10;
 
 #define EM_DECLARE_LAUNCHERS                                                               \

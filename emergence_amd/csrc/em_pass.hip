@@ -347,15 +347,15 @@ static hipError_t launch_ens_one(const EnsPassArgs& e, unsigned grid, hipStream_
 #define EM_FOR_TILE(CALL)                  \
     switch (cfg) {                         \
         case 0: return CALL(32, 8, 256);  \
-        case 1: return CALL(16, 16, 256);  \
-        case 2: return CALL(64, 8, 512);  \
-        case 3: return CALL(27, 8, 256);  \
-        case 4: return CALL(59, 4, 256);  \
-        case 5: return CALL(27, 4, 128);  \
-        case 6: return CALL(27, 2, 64);  \
-        case 7: return CALL(59, 1, 64);  \
-        case 8: return CALL(16, 4, 64);  \
-        case 9: return CALL(123, 4, 512);  \
+        case 1: return CALL(64, 8, 512);  \
+        case 2: return CALL(59, 1, 64);  \
+        case 3: return CALL(27, 2, 64);  \
+        case 4: return CALL(27, 8, 256);  \
+        case 5: return CALL(59, 4, 256);  \
+        case 6: return CALL(27, 4, 128);  \
+        case 7: return CALL(16, 16, 256);  \
+        case 8: return CALL(123, 4, 512);  \
+        case 9: return CALL(16, 4, 64);  \
         default: return hipErrorInvalidValue; \
     }
 template <int D, int MODE, class Args>

@@ -346,10 +346,10 @@ struct Grid {
     int default_cfg(int d, bool f32 = false) const {
         const int f = active(d == 2 ? 1 : 2) ? (d == 2 ? 1 : 2) : (d == 0 ? 1 : 0);
         const long long tiles = (n[d] + 26) / 27 * ((n[f] + 7) / 8) * (ncell / n[d] / n[f]);
-        if (tiles < 256) return 6;
-        if (f32 && mode != MODE_CENTRAL && tiles < 12000) return stride[d] == 1 && n[d] > 27 ? 7 : 3;
-        if (mode == MODE_HYBRID) return 3;
-        return tiles < 4096 ? (stride[d] == 1 ? 4 : 3) : 0;
+        if (tiles < 256) return TILE_27x2;
+        if (f32 && mode != MODE_CENTRAL && tiles < 12000) return stride[d] == 1 && n[d] > 27 ? TILE_59x1 : TILE_27x8;
+        if (mode == MODE_HYBRID) return TILE_27x8;
+        return tiles < 4096 ? (stride[d] == 1 ? TILE_59x4 : TILE_27x8) : TILE_32x8;
     }
 
     uint64_t faces_per_stage() const {
@@ -1157,7 +1157,7 @@ struct Ensemble {
     std::vector<Solver*> in;
     HostIo<5> io;  // of all instances, which transfer one after another
     int n = 0;
-    int mode, cfg = 4, precise = 1;
+    int mode, cfg = TILE_59x4, precise = 1;
     bool batched = true;
     double cfl;
     hipStream_t stream = nullptr;

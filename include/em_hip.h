@@ -82,9 +82,11 @@ int em_solver_destroy(em_solver* s);
  * build). */
 int em_solver_set_variant(em_solver* s, int32_t precise);
 
-/* Tile shape per axis (index into the library's tile table), and the
- * project autotuner that times every shape on the current state and keeps
- * the fastest per axis.  cfg_out may be NULL. */
+/* Tile shape per axis (index into the library's tile table: cells along the
+ * axis x pencils 32x8, 64x8, 59x1, 27x2, 27x8, 59x4, 27x4, 16x16, 123x4,
+ * 16x4), and the project autotuner that times every shape on the current
+ * state and keeps the fastest per axis.  Results do not depend on the shape.
+ * cfg_out may be NULL. */
 int em_solver_set_tiles(em_solver* s, const int32_t cfg[3]);
 int em_solver_autotune(em_solver* s, int32_t repeats, int32_t cfg_out[3]);
 

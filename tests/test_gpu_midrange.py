@@ -89,6 +89,32 @@ def test_residual_bits_in_and_outside_the_mid_range(em, kind, n, mode):
     assert np.array_equal(a[v].view(np.int64), b[v].view(np.int64)), "sign of a zero"
 
 
+@pytest.mark.parametrize("n", [(67, 9, 1), (12, 10, 70), (1, 70, 5)])
+@pytest.mark.parametrize("kind", ["fronts", "signed_zero", "small", "large", "near_vacuum", "cold", "outlier"])
+def test_hybrid_residuals_in_and_outside_the_mid_range(em, kind, n):
+    """Hybrid mode, where only part of a wave's lanes evaluate a midpoint.  The
+    sensor's logarithms differ from the host's by an ulp, which moves a blend
+    weight by at most 3 / (tol / 2) 16 ulp(ln) (below 1e-10 for |ln| < 128):
+    the bar is that share of the largest residual."""
+    bc = [["outflow", "outflow"], ["periodic", "periodic"], ["reflect", "outflow"]]
+    u = _state(n, kind)
+    g = em.HipSolver(n, (0, 0, 0), (1, 1, 1), u, mode="hybrid", bc=bc)
+    o = OracleSolver(n, (0, 0, 0), (1, 1, 1))
+    o.set_u(u)
+    o.set_opts(mode="hybrid")
+    for d in range(3):
+        for s in range(2):
+            o.set_bc(d, s, bc[d][s])
+    dt = o.dt_cfl()
+    a, sa = g.rhs(dt)
+    b, sb = o.rhs(dt)
+    a, b = o.interior(a), o.interior(b)
+    assert list(sa) == list(sb)
+    assert np.array_equal(np.isnan(a), np.isnan(b))
+    for k in range(5):
+        assert np.nanmax(np.abs(a[..., k] - b[..., k])) <= 1e-10 * np.nanmax(np.abs(b[..., k])), k
+
+
 @pytest.mark.parametrize("eos", [(5.0 / 3.0, 0.0, 0.0, 0.0), (4.4, 0.6, 0.0, 0.1), (1.3, 0.2, 0.3, -0.1)])
 def test_residual_bits_with_stiffened_and_covolume_gases(em, eos):
     n = (66, 11, 6)

@@ -15,7 +15,7 @@
 // padded array is many times the interior.  It also serves where the buffer
 // cannot be had.  In microseconds, host loop / device:
 //   in:  33x47 15/27, 64x64 23/31, 16^3 19/53, 1000x4x4 61/310,
-//        2x200x300 328/1291, 45x64x50 341/326, 512^2 833/339
+//        2x200x300 328/1291, 4x40000 515/727, 512^2 833/339
 //   out (seven variables): 64x48 25/36, 40x30x20 179/242, 1000x4x4 180/832
 #pragma once
 #include <hip/hip_runtime.h>
@@ -27,9 +27,9 @@
 namespace em {
 
 constexpr size_t kHostIoBytes = 256u << 20;
-// bytes read and written up to which the host loops stay in the caches (12 to
-// 17 GB/s; 3.5 GB/s at 80 MB)
-constexpr double kHostLoopBytes = 16e6;
+// interior bytes up to which the host loops stay in the caches (12 to 17 GB/s;
+// 3.5 GB/s at 40 MB)
+constexpr double kHostLoopBytes = 8e6;
 
 // Padded extents and ghost offsets of a mesh (int: a padded plane index fits)
 struct HostLayout {
@@ -110,27 +110,30 @@ struct HostIo {
         return true;
     }
     // Which side converts, by the time of either (microseconds, bytes per
-    // microsecond): a loop over the interior at 16 GB/s (23 in float, half
+    // microsecond).  in: a loop over the interior at 16 GB/s (23 in float, half
     // the bytes to write and copy) against the whole padded array at 30 GB/s
-    // and a kernel
+    // and a kernel.  The loop's staging array is new memory for each call where
+    // it is large: page faults at 16 GB/s (with them left out of the rule,
+    // 20 steps of a 65x99x27 state between upload and download took 6.7
+    // against 6.2 ms)
+    static double faults(double staged) { return std::max(0.0, staged - 1e6) / 16e3; }
     template <class Real>
     static bool in_on_host(const HostLayout& h) {
         const double ib = 8.0 * NV * h.ncell, pb = 8.0 * NV * h.len;
-        return ib * (1.0 + sizeof(Real) / 8.0) <= kHostLoopBytes &&
-               10.0 + ib / (sizeof(Real) == 4 ? 23e3 : 16e3) < 20.0 + pb / 30e3;
+        return ib <= kHostLoopBytes &&
+               10.0 + ib / (sizeof(Real) == 4 ? 23e3 : 16e3) + faults(ib * sizeof(Real) / 8.0) < 20.0 + pb / 30e3;
     }
     // out: interior planes are copied at 17 GB/s and scattered (8.2 together,
     // 15 in float) into zeros, or the padded array copied at 17.5; padded
-    // planes of doubles lose the transposition at 37 GB/s but save a kernel; in
-    // float they are half the bytes, which weighs more as long as the staging
-    // array is not mapped anew for each call (above 32 MB)
+    // planes of doubles lose the transposition at 37 GB/s but save a kernel, in
+    // float they are half the bytes
     template <class Real>
     static bool out_on_host(const HostLayout& h, bool padded) {
         const double ib = 8.0 * NV * h.ncell, pb = 8.0 * NV * h.len;
-        if (padded)
-            return sizeof(Real) == 4 ? pb <= 64e6 && pb / 27e3 < 5.0 + pb / 17.5e3 : pb / 11.9e3 < 5.0 + pb / 17.5e3;
-        return ib * (1.0 + sizeof(Real) / 8.0) <= kHostLoopBytes &&
-               10.0 + ib / (sizeof(Real) == 4 ? 15e3 : 8.2e3) + pb / 200e3 < 24.0 + pb / 17.5e3;
+        const double device = pb / 17.5e3, fault = faults((padded ? pb : ib) * sizeof(Real) / 8.0);
+        if (padded) return pb / (sizeof(Real) == 4 ? 27e3 : 11.9e3) + fault < 5.0 + device;
+        return ib <= kHostLoopBytes &&
+               10.0 + ib / (sizeof(Real) == 4 ? 15e3 : 8.2e3) + fault + pb / 200e3 < 24.0 + device;
     }
     template <class Real>
     hipError_t in_by_host(const HostLayout& h, const double* host, Real* dev, hipStream_t s) {

@@ -103,7 +103,7 @@ __device__ __forceinline__ void amr_item(const AmrPassArgsT<Real>& pa, long long
     // amr.rs:1254; formed in double from the device dt and rounded to Real
     const double lam = pa.ndim_pos > 0.0 ? pa.ndim_pos * dtv / (double)dx : 0.0;
     tile_faces<D, MODE, NT>(L, tid, true, B, Pv, 0, 0, B, B, e, Real(lam), pa.tol, a.bd[(D + 1) % 3] == 1,
-                            a.bd[(D + 2) % 3] == 1, n_shock, scnt, [](int, int, int) { return Real(0.0); }, [] {});
+                            a.bd[(D + 2) % 3] == 1, n_shock, scnt, [] {});
     // ---- residual and boundary face fluxes
     for (int it = tid; it < B * P; it += NT) {
         int c, p;

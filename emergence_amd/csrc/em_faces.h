@@ -23,8 +23,9 @@
 // either may evaluate one that the other does not need.  So that a fallback
 // there is counted once whatever the tiles, the left tile counts what it
 // evaluates, and this one what the left one does not; the weights of the faces
-// -4 .. -1 that this takes are evaluated for such a fallback only (with every
-// tile's other weights they cost 3% of a Hybrid residual).
+// -4 .. -1 that this takes are evaluated for such a fallback only, behind the
+// other phases (with every tile's other weights they cost 3% of a Hybrid
+// residual, this way 1.5%).
 #pragma once
 #include "em_device.h"
 #include "em_types.h"
@@ -67,6 +68,7 @@ struct Tile {
     Real sf[5][P];      // flux of face 0
     Real ss[2][HYB ? C * P : 1];
     Real sth[HYB ? TH * P : 1];
+    unsigned late[HYB && CUT ? P : 1];  // fallbacks of the midpoints 0 .. 3 that late_fallbacks decides on
 };
 
 // lanes of the wave that satisfy c (called where the wave is whole)
@@ -90,6 +92,37 @@ __device__ __forceinline__ R blend_weight(R tol, LD&& ld) {
     return isfinite(r) ? x * x * (R(3.0) - R(2.0) * x) : R(1.0);
 }
 
+// Counts the fallbacks in L.late that the tile before did not: those whose
+// faces -4 .. -1 all have weight zero.  left_sensor(p, h, k) is sensor k of the
+// cell h - 2 before pencil p's tile.  (Every thread calls it, after
+// tile_faces; apart from the midpoints, whose loop it would slow down.)
+template <class R, class TL, class SEN>
+__device__ __forceinline__ void late_fallbacks(TL& L, int tid, R tol, unsigned (&scnt)[3], SEN&& left_sensor) {
+    const unsigned late = tid < TL::P ? L.late[tid] : 0;
+    if (late == 0) return;
+    R x[2][2] = {};
+#pragma unroll 1
+    for (int i = 0; i < 4; ++i) {
+        const R y = left_sensor(tid, i & 1, i >> 1);
+        x[0][0] = i == 0 ? y : x[0][0];
+        x[1][0] = i == 1 ? y : x[1][0];
+        x[0][1] = i == 2 ? y : x[0][1];
+        x[1][1] = y;
+    }
+    unsigned n = 0;
+    bool zero = true;  // the weights of the faces f .. -1
+#pragma unroll 1
+    for (int f = -1; f >= -4; --f) {
+        zero = zero && !(blend_weight(tol, [&](int j, int k) {
+                             const int c = f + 2 + j;
+                             return c == -2 ? x[0][k] : c == -1 ? x[1][k] : L.ss[k][TL::at(c, tid)];
+                         }) > R(0.0));
+        // midpoint m = f + 4 reaches down to face f
+        n += zero && (late >> (f + 4) & 1) ? 1 : 0;
+    }
+    if (n) atomicAdd(&scnt[1], n);
+}
+
 // On entry (after a barrier): the tile's cells are in sw, sre and ss.  On
 // exit (after a barrier): the flux of face f = 1 .. Tv is sm[k][mt(f - 1, p)],
 // of face 0 sf[k][p].  first: nothing was taken over.  Counters of midpoints
@@ -97,14 +130,12 @@ __device__ __forceinline__ R blend_weight(R tol, LD&& ld) {
 // shock-path faces are counted per wave (a scalar register), fallbacks and
 // limited faces, which are few, in scnt[1] and scnt[2].  before_last() is
 // called once the faces are in registers, ahead of the last two barriers: the
-// place to issue the loads of the phase that follows.  left_sensor(p, h, k) is
-// sensor k of the cell h - 2 before pencil p's tile (Hybrid, CUT, s0 > 0).
-// zero1, zero2: the axes of the transverse velocities (D+1) % 3 and (D+2) % 3
+// place to issue the loads of the phase that follows.  zero1, zero2: the axes of the transverse velocities (D+1) % 3 and (D+2) % 3
 // are inactive (see midpoint_flux_mid).
-template <int D, int MODE, int NT, class R, class TL, class SEN, class PRE>
+template <int D, int MODE, int NT, class R, class TL, class PRE>
 __device__ __forceinline__ void tile_faces(TL& L, int tid, bool first, int Tv, int Pv, int c0, int s0, int s1, int nD,
                                            const EosT<R>& e, R lam, R tol, bool zero1, bool zero2,
-                                           unsigned& n_shock, unsigned (&scnt)[3], SEN&& left_sensor, PRE&& before_last) {
+                                           unsigned& n_shock, unsigned (&scnt)[3], PRE&& before_last) {
     constexpr int T = TL::T, P = TL::P;
     constexpr bool HYB = MODE == MODE_HYBRID;
     constexpr bool CEN = MODE == MODE_CENTRAL;
@@ -153,24 +184,10 @@ __device__ __forceinline__ void tile_faces(TL& L, int tid, bool first, int Tv, i
                 const int j = c0 - 3 + m;  // global midpoint index
                 bool own = (s0 == 0 || j >= s0) && (s1 == nD || j < s1);
                 if constexpr (HYB && TL::CUT) {
-                    own = s0 == 0 || m > 4 || !(L.sth[TL::tt(0, p)] > R(0.0));
-                    if (own && s0 > 0 && m < 4) {
-                        R x[2][2] = {};  // sensors of the cells -2 and -1
-#pragma unroll 1
-                        for (int i = 0; i < 4; ++i) {
-                            const R y = left_sensor(p, i & 1, i >> 1);
-                            x[0][0] = i == 0 ? y : x[0][0];
-                            x[1][0] = i == 1 ? y : x[1][0];
-                            x[0][1] = i == 2 ? y : x[0][1];
-                            x[1][1] = y;
-                        }
-#pragma unroll 1
-                        for (int f = m - 4; f < 0; ++f)
-                            own = own && !(blend_weight(tol, [&](int j, int k) {
-                                               const int c = f + 2 + j;
-                                               return c == -2 ? x[0][k] : c == -1 ? x[1][k] : L.ss[k][TL::at(c, p)];
-                                           }) > R(0.0));
-                    }
+                    // with a weight at face 0 the left tile has evaluated it
+                    own = s0 == 0 || m >= 4 || L.sth[TL::tt(0, p)] > R(0.0);
+                    if (!own) atomicOr(&L.late[p], 1u << m);
+                    own = own && (s0 == 0 || m > 4 || !(L.sth[TL::tt(0, p)] > R(0.0)));
                 }
                 if (own) atomicAdd(&scnt[1], 1u);
             }

@@ -120,6 +120,7 @@ __device__ __forceinline__ void axis_segment(const PassArgsT<Real>& a, int bid, 
     const long long nc = a.ncell;
     const EosT<Real> e = a.eos;
     if (tid < 3) scnt[tid] = 0;
+    if (HYB && tid < P) L.late[tid] = 0;
     // read together and tested behind the first tile's loads: one round trip
     const int active = a.sc->active;
     const double dt_d = wave_uniform(a.sc->dt);
@@ -186,16 +187,7 @@ __device__ __forceinline__ void axis_segment(const PassArgsT<Real>& a, int bid, 
         const long long idx = base + (long long)p * sF + (long long)(c0 + c) * sD;
         Real r[5], u0[5], us[5];
         tile_faces<D, MODE, NT>(L, tid, first, Tv, Pv, c0, s0, s1, nD, e, lam, a.tol, !a.active[(D + 1) % 3],
-                                !a.active[(D + 2) % 3], n_shock, scnt,
-                                [&](int p, int h, int k) {
-                                    Real u[5], w[5];
-                                    const long long i = base + (long long)p * sF + (long long)(c0 - 7 + h) * sD;
-#pragma unroll
-                                    for (int q = 0; q < 5; ++q) u[q] = a.U[q * nc + i];
-                                    to_prim(e, u, w);
-                                    return log(fmax(k ? w[4] + e.p_inf : w[0], Real(1e-300)));
-                                },
-                                [&] {
+                                !a.active[(D + 2) % 3], n_shock, scnt, [&] {
 #pragma unroll
                                     for (int k = 0; k < 5; ++k) {
                                         r[k] = a.first || !mine ? Real(0.0) : a.R[k * nc + idx];
@@ -241,7 +233,17 @@ __device__ __forceinline__ void axis_segment(const PassArgsT<Real>& a, int bid, 
                 }
             }
         }
-        if constexpr (HYB) break;  // one tile (cut_segments)
+        if constexpr (HYB) {
+            late_fallbacks(L, tid, a.tol, scnt, [&](int p, int h, int k) {
+                Real u[5], w[5];
+                const long long i = base + (long long)p * sF + (long long)(c0 - 7 + h) * sD;
+#pragma unroll
+                for (int q = 0; q < 5; ++q) u[q] = a.U[q * nc + i];
+                to_prim(e, u, w);
+                return log(fmax(k ? w[4] + e.p_inf : w[0], Real(1e-300)));
+            });
+            break;  // one tile (cut_segments)
+        }
         // the cells the next tile takes over
         if (c0 + T < s1) {
             for (int it = tid; it < TL::HC * P; it += NT) {

@@ -167,7 +167,7 @@ __device__ __forceinline__ double rcp_volume(const Eos& e, double rho, double vb
 // is finite; no division.  With d = (E - |m|^2 / 2 rho - rho q - p_inf (1 -
 // rho b)) rho = rho^2 (v - b) (p + p_inf) / (gamma - 1), the test asks for
 // d > margin times the sum of the terms' magnitudes; the rounding of either
-// evaluation is below 1e-5 of that slack.
+// evaluation is below 1e-5 of that slack in double and a tenth of it in float.
 template <class R>
 __device__ __forceinline__ bool clearly_admissible(const EosT<R>& e, const R q[5]) {
     const R rho = q[0];
@@ -498,11 +498,12 @@ __device__ __forceinline__ void weno5z_pair(const double v[6], double& left, dou
 // value k of cell j read through ld(j, k): the same flux, or false (and no
 // flux) where some operand is outside, or a reconstruction inadmissible: the
 // caller then evaluates midpoint_flux.  The pass is bound by its FP64
-// instruction count (VALU 87% busy), much of it divisions: 61 per midpoint,
-// here 6 in the general form and the rest through shared reciprocals.  With
-// the load phase's and the limiter's divisions (to_prim_v,
+// instruction count (VALU 86% busy), much of it divisions: 61 per midpoint,
+// here 3 in the general form (hllc_flux) and the rest through shared
+// reciprocals.  With the load phase's and the limiter's divisions (to_prim_v,
 // clearly_admissible) the 256^3 Weno x pass went from 2,544 to 2,033 VALU
-// instructions per cell, the three passes from 4.29 to 3.56 ms.
+// instructions per cell in the same tiles, the three passes from 4.29 to 3.56
+// ms (1,857 and 3.11 ms in segments, em_pass.hip).
 //   * l4un = -l0un and l44 = l04 = -l14 / 2 exactly (powers of two and signs),
 //     so the fields 0, 1 and 4 need two products per cell.
 //   * zero1, zero2: the axes of the transverse velocities t1, t2 are

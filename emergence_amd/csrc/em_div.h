@@ -30,12 +30,9 @@ struct Mid<double> {
     static constexpr double margin = 1e-9;        // relative slack of clearly_admissible (rounding: about 1e-15)
 };
 template <>
-struct Mid<float> {
+struct Mid<float> {  // clearly_admissible only
     static constexpr float lo = 0x1p-40f, hi = 0x1p+40f;
-    static constexpr float tiny = 0x1p-80f;
-    static constexpr float huge = 0x1p+110f;
-    static constexpr float beta_max = 0x1p+100f;
-    static constexpr float margin = 1e-3f;
+    static constexpr float margin = 1e-3f;  // (rounding: up to 1e-4 as gamma nears 1.01)
 };
 
 // x within [lo, hi] (false for NaN)

@@ -25,10 +25,10 @@
 // EM_VARIANT=fast with FMA contraction; EM_MODE = 0 hybrid, 1 weno,
 // 2 central.  Kernels ask for 4 waves per SIMD (<= 128 VGPRs).
 //
-// Bound by FP64 instruction issue (VALU 81 to 85% busy).  256^3 Weno, x, y and
-// z pass of a step: 1.58, 1.60, 1.76 ms with independent 59-cell tiles and
-// general divisions (2,544 VALU instructions per cell along x), 1.03, 1.04,
-// 1.13 ms now (about 1,800).  Code size counts: a version that inlined the
+// Bound by FP64 instruction issue (VALU 85 to 86% busy).  256^3 Weno, x, y and
+// z pass of a step: 1.41 to 1.45 and 1.57 to 1.65 ms (z) with independent
+// 59-cell tiles and general divisions (2,544, 2,551 and 2,768 VALU
+// instructions per cell), 1.03, 1.05, 1.23 ms now (1,857, 1,881 and 2,256).  Code size counts: a version that inlined the
 // boundary images three times (59 KB) ran 20% slower than this one.
 #include <hip/hip_runtime.h>
 

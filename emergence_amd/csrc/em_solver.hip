@@ -313,9 +313,11 @@ struct Grid {
         return a;
     }
 
-    // Segments of a pass along d with tile shape cfg.  Long segments share most (see em_faces.h); the launch
-    // still has to fill the GPU (256 CUs of 16 waves) twice over so that its
-    // last round weighs little.  Hybrid: single tiles.
+    // Segments of a pass along d with tile shape cfg.  Long segments share
+    // most (see em_faces.h); the launch still has to fill the GPU (256 CUs of
+    // 16 waves) twice over so that its last round weighs little.  Hybrid:
+    // single tiles.  An ensemble's instances are cut by the same rule, each as
+    // if alone.
     template <class Real>
     static void cut_segments(PassArgsT<Real>& a, int d, int mode, int cfg) {
         const long long groups = (long long)a.ngroup * a.n[a.slow_axis];

@@ -65,7 +65,8 @@ struct PassArgsT {
 using PassArgs = PassArgsT<double>;
 
 // Ensemble pass: per-instance pass arguments, the prefix sums of the
-// instances' segment counts and each segment's instance (ninst + 1 entries; total = prefix[ninst]).
+// instances' segment counts (ninst + 1 entries; total = prefix[ninst]) and
+// each segment's instance.
 struct EnsPassArgs {
     const PassArgs* args;
     const long long* prefix;

@@ -18,6 +18,8 @@ constexpr TileCfg kTileCfgs[] = {{32, 8, 256}, {64, 8, 512}, {59, 1, 64}, {27, 2
                                  {59, 4, 256}, {27, 4, 128}, {16, 16, 256}, {123, 4, 512}, {16, 4, 64}};
 enum : int { TILE_32x8 = 0, TILE_59x1 = 2, TILE_27x2 = 3, TILE_27x8 = 4, TILE_59x4 = 5 };
 constexpr int kNumTileCfgs = 10;
+// a launch of more threads runs a part of them and reports no error
+constexpr long long kMaxLaunchThreads = 0xffffffffll;
 
 #define EM_DECLARE_LAUNCHERS                                                               \
     hipError_t launch_pass_hybrid(int d, int cfg, const PassArgs& a, hipStream_t s);      \

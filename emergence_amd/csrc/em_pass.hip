@@ -319,7 +319,9 @@ __global__ __launch_bounds__(NT) __attribute__((amdgpu_waves_per_eu(EM_WAVES_PER
 // whether the pass axis is contiguous (the last axis always is).
 template <int D, int MODE, int T, int P, int NT>
 static hipError_t launch_one(const PassArgs& a, hipStream_t s) {
-    const dim3 grid((unsigned)((long long)a.nseg * a.ngroup * a.n[a.slow_axis]));
+    const long long blocks = (long long)a.nseg * a.ngroup * a.n[a.slow_axis];
+    if (blocks * NT > kMaxLaunchThreads) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)blocks);
     if (D == 2 || a.dfast)
         hipLaunchKernelGGL((axis_pass<D, MODE, T, P, true, NT>), grid, dim3(NT), 0, s, a);
     else
@@ -328,7 +330,9 @@ static hipError_t launch_one(const PassArgs& a, hipStream_t s) {
 }
 template <int D, int MODE, int T, int P, int NT>
 static hipError_t launch_one(const PassArgsT<float>& a, hipStream_t s) {
-    const dim3 grid((unsigned)((long long)a.nseg * a.ngroup * a.n[a.slow_axis]));
+    const long long blocks = (long long)a.nseg * a.ngroup * a.n[a.slow_axis];
+    if (blocks * NT > kMaxLaunchThreads) return hipErrorInvalidValue;
+    const dim3 grid((unsigned)blocks);
     if (D == 2 || a.dfast)
         hipLaunchKernelGGL((axis_pass_f32<D, MODE, T, P, true, NT>), grid, dim3(NT), 0, s, a);
     else

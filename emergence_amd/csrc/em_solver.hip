@@ -320,14 +320,30 @@ struct Grid {
     // if alone.
     template <class Real>
     static void cut_segments(PassArgsT<Real>& a, int d, int mode, int cfg) {
-        const long long groups = (long long)a.ngroup * a.n[a.slow_axis];
         const TileCfg tc = kTileCfgs[cfg];
-        const long long resident = 256ll * 16 * 64 / tc.NT;
-        const int ntile = (a.n[d] + tc.T - 1) / tc.T;
-        const long long want = (2 * resident + groups - 1) / groups;
-        const int per = mode == MODE_HYBRID ? 1 : (int)std::max<long long>(1, ntile / std::min<long long>(want, ntile));
-        a.seg = per * tc.T;
+        a.seg = tc.T * tiles_per_segment((a.n[d] + tc.T - 1) / tc.T, (long long)a.ngroup * a.n[a.slow_axis], mode, tc.NT);
         a.nseg = (a.n[d] + a.seg - 1) / a.seg;
+    }
+    static int tiles_per_segment(int ntile, long long groups, int mode, int nt) {
+        const long long resident = 256ll * 16 * 64 / nt;
+        const long long want = (2 * resident + groups - 1) / groups;
+        return mode == MODE_HYBRID ? 1 : (int)std::max<long long>(1, ntile / std::min<long long>(want, ntile));
+    }
+
+    // Threads of the launch along d with tile shape cfg (a launch of 2^32 or
+    // more runs a part of them, without an error).
+    long long pass_threads(int d, int cfg) const {
+        const TileCfg tc = kTileCfgs[cfg];
+        const int f = fast_axis(d);
+        const long long groups = (n[f] + tc.P - 1) / tc.P * (ncell / n[d] / n[f]);
+        const int ntile = (int)((n[d] + tc.T - 1) / tc.T);
+        const int per = tiles_per_segment(ntile, groups, mode, tc.NT);
+        return (ntile + per - 1) / per * groups * tc.NT;
+    }
+    // transverse axis of a workgroup's pencils
+    int fast_axis(int d) const {
+        const int inner = d == 2 ? 1 : 2;
+        return active(inner) ? inner : d == 0 ? 1 : 0;
     }
 
     // Tile shape of axis d before any autotuning, by the number of 27 x 8
@@ -345,8 +361,14 @@ struct Grid {
     // 32-cell tiles; Hybrid z axis 189 against 281 in 27-cell tiles; 160^3
     // Weno, 19,200 tiles: 200-228 us in 32-cell tiles against 221-251).  Pencils
     // of one tile stay with the 27-cell shape (300x20x20, z: 23 against 28 us).
+    // Meshes too long for one launch in those shapes (a line of 4.5e8 cells in
+    // 27 x 8 tiles) take 59 x 1, which wastes the fewest threads (3.9e9).
     int default_cfg(int d, bool f32 = false) const {
-        const int f = active(d == 2 ? 1 : 2) ? (d == 2 ? 1 : 2) : (d == 0 ? 1 : 0);
+        const int c = preferred_cfg(d, f32);
+        return pass_threads(d, c) <= kMaxLaunchThreads ? c : TILE_59x1;
+    }
+    int preferred_cfg(int d, bool f32) const {
+        const int f = fast_axis(d);
         const long long tiles = (n[d] + 26) / 27 * ((n[f] + 7) / 8) * (ncell / n[d] / n[f]);
         if (tiles < 256) return TILE_27x2;
         if (f32 && mode != MODE_CENTRAL && tiles < 12000) return stride[d] == 1 && n[d] > 27 ? TILE_59x1 : TILE_27x8;
@@ -696,7 +718,7 @@ struct SolverCore : Grid {
             double best = 1e300;
             int bestc = cfg[d];
             for (int c = 0; c < kNumTileCfgs; ++c) {
-                if (kTileCfgs[c].T > 2 * n[d] && c != 0) continue;
+                if ((kTileCfgs[c].T > 2 * n[d] && c != 0) || pass_threads(d, c) > kMaxLaunchThreads) continue;
                 cfg[d] = c;
                 PassArgsT<Real> a = pass_args(d);
                 a.U = U[0];
@@ -1830,9 +1852,7 @@ static void rhs_noalloc(const Grid& G, int precise, double stage_dt, const doubl
     if (sizeof(DevScalars) > kNoAllocScratchBytes) throw Error(EM_ERR_ARG, "scratch too small for the device scalars");
     for (int d = 0; d < 3; ++d) {
         if (!G.active(d)) continue;
-        const PassArgs a = G.pass_args(d, nullptr);
-        const long long nblk = (long long)a.nseg * a.ngroup * a.n[a.slow_axis];
-        if (nblk > 0x7fffffffll) throw Error(EM_ERR_ARG, "mesh too large for one axis-pass launch");
+        if (G.pass_threads(d, G.cfg[d]) > kMaxLaunchThreads) throw Error(EM_ERR_ARG, "mesh too large for one axis-pass launch");
     }
     DevScalars* sc = noalloc_scratch();
     hipLaunchKernelGGL(k_noalloc_reset, dim3(1), dim3(kSlots), 0, st, sc);
